@@ -1184,7 +1184,7 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       plastic();
     }
   }
-  if (!loc) L("locate", [&] { launch_locate_step<D>(M, P, S, scan, st); });
+  if (!loc) L("locate", [&] { launch_locate_step<D>(!ordered, M, P, S, scan, st); });
   L("locate_scan", [&] { launch_locate_scan<D>(M, P, S, scan, nullptr, c->locate_all ? 0 : 1, st); });
   L("step_end", [&] { launch_step_end(S, st); });
 }

@@ -19,8 +19,9 @@ void launch_locate_init(const Mesh& M, const Particles& P, Status* S, int* scan_
                         const int* hint, hipStream_t st);
 // Per-step locate of an isoparametric mesh (current cell, neighbours, else the
 // scan queue); the step kernels locate Cartesian meshes themselves.
+// fast: fast mode's cheaper inverse of hex8 cells (same point to 2e-13).
 template <int D>
-void launch_locate_step(const Mesh& M, const Particles& P, Status* S, int* scan_list,
+void launch_locate_step(bool fast, const Mesh& M, const Particles& P, Status* S, int* scan_list,
                         hipStream_t st);
 // Affine velocity updates (APIC, ASFLIP, TPIC): the mapping matrices (and
 // ASFLIP's beta) before G2P; the matrix of the next particle-to-grid
