@@ -104,6 +104,7 @@ struct mpmx_ctx {
   // isoparametric mesh: local coordinates by transform_real_to_unit_cell
   // (cell.tcc:617-828), located by a kernel of its own each step
   bool iso = false;
+  bool box = false;  // Mesh::box
   // instances (batched runs): cell ranges, cell -> instance
   int64_t ninst = 0;
   DBuf<int> d_cell_inst;
@@ -257,6 +258,7 @@ struct mpmx_ctx {
     M.cell_inst = ninst > 0 ? d_cell_inst.p : nullptr;
     M.inst_begin = ninst > 0 ? d_inst_begin.p : nullptr;
     M.iso = iso ? 1 : 0;
+    M.box = box ? 1 : 0;
     return M;
   }
   Particles parts() const {
@@ -553,6 +555,7 @@ Material make_material(const double* p) {
   dmath::sincos(m.phi_peak, &m.sphi, &m.cphi);
   m.tphi = m.sphi / m.cphi;
   m.tpsi = dmath::tan(m.psi_peak);
+  fast_angle_constants(m.sphi, m.cphi, m.tpsi, m.fk);
   // initialise_state_variables (mohr_coulomb.tcc:85-111)
   m.sv0[SV_YIELD] = 0;
   m.sv0[SV_PHI] = m.phi_peak;
@@ -1070,6 +1073,18 @@ struct Launcher {
   }
 };
 
+// Whether the stress kernels use fast mode's regrouped arithmetic
+// (mpmx_fast.h): in 3D without a stress rate. There fast mode's nodal sums
+// (four and more atomic contributions per node) already differ from run to
+// run by rounding, which a plastic run magnifies, and 10 + 10 steps of the
+// 2.1M-particle collapse differ as much between two runs of one build as
+// between the two arithmetics (velocities 1e-13 to 6e-9 over seeds). In 2D a
+// node has two contributions as a rule, runs repeat to 1e-12, and the
+// reference's arithmetic is kept.
+bool fast_stress(const mpmx_ctx* c) {
+  return c->dim == 3 && !(c->flags & MPMX_ORDERED) && !c->any_rate;
+}
+
 template <int D>
 void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
                   const StepBuffers& B) {
@@ -1104,8 +1119,10 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       launch_fn_eval(c->d_fns.p, c->d_fn_data.p, (int)c->fns.size(), S, A.dt, B.fnval, st);
     });
   // the Mohr-Coulomb return mappings deferred by the stress kernels
+  // (3D fast mode without a stress rate completes them in its own kernels)
+  const bool own = fast_stress(c);
   auto plastic = [&] {
-    if (c->any_mc) L("mc_plastic", [&] { launch_plastic(P, mats, S, st); });
+    if (c->any_mc && !own) L("mc_plastic", [&] { launch_plastic(P, mats, S, st); });
   };
   // affine velocity updates (APIC, ASFLIP, TPIC): the transfer matrix before
   // each particle-to-grid map, the mapping matrix before grid-to-particle
@@ -1131,23 +1148,23 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
     affine();
     if (c->scheme == USF) {
       L("gather_mass_momentum", [&] { launch_gather<D>(GK_MV_VEL, M, P, Nd, A, S, perm, cs, ce, st); });
-      L("stress", [&] { launch_stress<D>(false, M, P, Nd, mats, A, S, scan, st); });
+      L("stress", [&] { launch_stress<D>(own, false, M, P, Nd, mats, A, S, scan, st); });
       plastic();
       L("gather_forces", [&] { launch_gather<D>(GK_F_ACC, M, P, Nd, A, S, perm, cs, ce, st); });
       mapping();
-      L("g2p_locate", [&] { launch_g2p<D>(false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
+      L("g2p_locate", [&] { launch_g2p<D>(own, false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
     } else if (c->scheme == USL) {
       L("gather_all", [&] { launch_gather<D>(GK_ALL_VEL_ACC, M, P, Nd, A, S, perm, cs, ce, st); });
       mapping();
-      L("g2p_stress_locate", [&] { launch_g2p<D>(true, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
+      L("g2p_stress_locate", [&] { launch_g2p<D>(own, true, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
       plastic();
     } else {
       L("gather_all", [&] { launch_gather<D>(GK_ALL_VEL_ACC, M, P, Nd, A, S, perm, cs, ce, st); });
       mapping();
-      L("g2p", [&] { launch_g2p<D>(false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
+      L("g2p", [&] { launch_g2p<D>(own, false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
       affine();
       L("gather_momentum", [&] { launch_gather<D>(GK_MOM_VEL, M, P, Nd, A, S, perm, cs, ce, st); });
-      L("stress_locate", [&] { launch_stress<D>(loc, M, P, Nd, mats, A, S, scan, st); });
+      L("stress_locate", [&] { launch_stress<D>(own, loc, M, P, Nd, mats, A, S, scan, st); });
       plastic();
     }
   } else {
@@ -1159,13 +1176,13 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_acceleration", [&] { launch_node<D>(ND_ACC | ND_ZERO_ALL, M, Nd, A, S, st); });
       mapping();
-      L("g2p_locate", [&] { launch_g2p<D>(false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
+      L("g2p_locate", [&] { launch_g2p<D>(own, false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
     } else if (c->scheme == USL) {
       L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, skey, perm, st); });
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_update", [&] { launch_node<D>(ND_INIT | ND_VEL | ND_ACC | ND_ZERO_ALL, M, Nd, A, S, st); });
       mapping();
-      L("g2p_stress_locate", [&] { launch_g2p<D>(true, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
+      L("g2p_stress_locate", [&] { launch_g2p<D>(own, true, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
       plastic();
     } else {
       L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, skey, perm, st); });
@@ -1173,14 +1190,14 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       L("node_update", [&] { launch_node<D>(ND_INIT | ND_VEL | ND_ACC | ND_ZERO_MOM, M, Nd, A, S, st); });
       if (aff) {  // G2P, then the affine momentum map with the new positions
         mapping();
-        L("g2p", [&] { launch_g2p<D>(false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
+        L("g2p", [&] { launch_g2p<D>(own, false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
         affine();
         L("p2g_momentum", [&] { launch_p2g<D>(P2G_MOM, c->chunk, M, P, Nd, A, S, skey, perm, st); });
       } else {
         L("g2p_momentum_scatter", [&] { launch_g2p_scatter<D>(c->chunk, M, P, Nd, A, c->vu, S, skey, perm, st); });
       }
       L("node_velocity", [&] { launch_node<D>(ND_VEL | ND_ZERO_ALL, M, Nd, A, S, st); });
-      L("stress_locate", [&] { launch_stress<D>(loc, M, P, Nd, mats, A, S, scan, st); });
+      L("stress_locate", [&] { launch_stress<D>(own, loc, M, P, Nd, mats, A, S, scan, st); });
       plastic();
     }
   }
@@ -1704,6 +1721,7 @@ int mpmx_set_mesh(mpmx_ctx* c, int64_t nnodes, const double* coords, int64_t nce
   // geometry
   std::vector<double> centroid(d * ncells), len(d * ncells), two_mean(ncells), dndx_c(ncells * nn * d);
   c->cell_volume.assign(ncells, 0.);
+  c->box = true;
   static const int q_sides[4][2] = {{0, 1}, {1, 2}, {2, 3}, {3, 0}};
   static const int h_sides[12][2] = {{0, 1}, {1, 2}, {2, 3}, {3, 0}, {4, 5}, {5, 6},
                                      {6, 7}, {7, 4}, {0, 4}, {1, 5}, {2, 6}, {3, 7}};
@@ -1728,6 +1746,17 @@ int mpmx_set_mesh(mpmx_ctx* c, int64_t nnodes, const double* coords, int64_t nce
     len[0 * ncells + ci] = norm_diff(d, X[0], X[1]);
     len[1 * ncells + ci] = norm_diff(d, X[1], X[2]);
     if (d == 3) len[2 * ncells + ci] = norm_diff(d, X[1], X[5]);
+    // a box in the element's node order: every node at its corner to 4 ulp of
+    // the largest coordinate (structured grids round there)
+    for (int i = 0; i < nn && c->box; ++i) {
+      const int l = i & 3;
+      const bool up[3] = {l == 1 || l == 2, l >= 2, i >= 4};
+      for (int k = 0; k < d; ++k) {
+        const double o = X[0][k], x = o + (up[k] ? len[k * ncells + ci] : 0.);
+        const double big = std::max(std::fabs(o), std::fabs(x));
+        if (std::fabs(X[i][k] - x) > 4 * 2.3e-16 * big) c->box = false;
+      }
+    }
     c->cell_volume[ci] = d == 2 ? quad_volume(X) : hex_volume(X);
     if (!(c->cell_volume[ci] > 0))
       throw ApiError(MPMX_E_ARG, "Negative or zero volume cell, misconfigured cell: " + std::to_string(ci));

@@ -5,6 +5,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 namespace mpmx {
@@ -33,6 +34,8 @@ struct Material {
   // sin, cos, tan of the peak friction angle and tan of the peak dilation
   // angle, by the same functions as the per-particle evaluation
   double sphi, cphi, tphi, tpsi;
+  // fast mode's constants of the peak angles (fast_angle_constants)
+  double fk[8];
   // MohrCoulomb without softening whose particles all hold the initial
   // friction, dilation, cohesion and tension cutoff (state variables 1-4,
   // which nothing changes then): the kernels take them from sv0
@@ -40,6 +43,25 @@ struct Material {
 };
 
 enum { RATE_NONE = 0, RATE_JAUMANN = 1, RATE_GREEN_NAGHDI = 2 };
+
+// Constants of a friction / dilation angle pair that the yield functions and
+// the potential use: tan phi, 1 / (sqrt(3) cos phi), n = (1 + sin phi) / (1 -
+// sin phi), sqrt(n), sqrt(1 + n^2) + n, (3 - sin phi) / (6 cos phi), the
+// potential's eccentricity, tan psi.
+__host__ __device__ inline void fast_angle_constants(double sphi, double cphi, double tpsi,
+                                                     double* fk) {
+  fk[0] = sphi / cphi;
+  fk[1] = 1. / (1.7320508075688772 * cphi);
+  fk[2] = (1. + sphi) / (1. - sphi);
+  fk[3] = sqrt(fk[2]);
+  fk[4] = sqrt(1. + fk[2] * fk[2]) + fk[2];
+  fk[5] = (3. - sphi) / (6 * cphi);
+  double e = (3. - sphi) / (3. + sphi);
+  if (e <= 0.5) e = 0.5 + 1.E-10;
+  if (e > 1.) e = 1.;
+  fk[6] = e;
+  fk[7] = tpsi;
+}
 
 // Nodal constraint record, referenced by Nodes::cons[node] (-1: none).
 struct NodeCons {
@@ -90,6 +112,9 @@ struct Mesh {
   // Null for a single mesh.
   const int* cell_inst;
   const int64_t* inst_begin;
+  // every cell is an axis-aligned rectangle / box in the element's node order
+  // with sides len: dN/dx of fast mode needs no node coordinates
+  int box;
   // isoparametric mesh (the reference's "isoparametric" mesh key): local
   // coordinates by the inverse of the element map, else the Cartesian formula
   int iso;

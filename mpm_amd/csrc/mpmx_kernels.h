@@ -51,8 +51,10 @@ template <int D>
 void launch_stress_scatter(int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
                            const Material* mats, const StepArgs& A, const Status* S,
                            const int* skey, const int* perm, hipStream_t st);
+// fast: fast mode without a stress rate; the kernels then complete their own
+// return mappings (launch_plastic is not needed).
 template <int D>
-void launch_stress(bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
+void launch_stress(bool fast, bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
                    const Material* mats, const StepArgs& A, Status* S, int* scan_list,
                    hipStream_t st);
 // Particle tractions onto the nodes' external force (fast mode; P.ntr > 0).
@@ -64,7 +66,7 @@ void launch_traction_scatter(const Mesh& M, const Particles& P, const Nodes& Nd,
 // stress or state variables.
 void launch_plastic(const Particles& P, const Material* mats, const Status* S, hipStream_t st);
 template <int D>
-void launch_g2p(bool stress, bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
+void launch_g2p(bool fast, bool stress, bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
                 const Material* mats, const StepArgs& A, int vu, Status* S, int* scan_list,
                 hipStream_t st);
 template <int D>

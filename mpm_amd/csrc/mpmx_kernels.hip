@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include "mpmx_device.h"
+#include "mpmx_fast.h"
 #include "mpmx_kernels.h"
 
 namespace mpmx {
@@ -47,6 +48,8 @@ static constexpr int kStressBlock = 128;
 #define MPMX_PLASTIC_WAVES 2
 #endif
 #define MPMX_PLASTIC_ATTR __attribute__((amdgpu_waves_per_eu(MPMX_PLASTIC_WAVES)))
+
+#define MPMX_WAVES(n) __attribute__((amdgpu_waves_per_eu(n)))
 
 MPMX_DEV void atomic_add(double* p, double v) { unsafeAtomicAdd(p, v); }
 
@@ -366,6 +369,24 @@ MPMX_DEV void stress_strain(const Mesh& M, const Particles& P, const Material* m
   }
 #pragma unroll
   for (int k = 0; k < 6; ++k) stream_st(&P.stress[k * np + p], s[k]);
+}
+
+// Velocity update of one component: v0 and the interpolated nodal velocity sv
+// and acceleration sa give the new velocity v and the velocity dx that moves
+// the particle.
+MPMX_DEV void update_velocity(int vu, const StepArgs& A, double beta, double v0, double sv,
+                              double sa, double* v, double* dx) {
+  *dx = sv;
+  if (vu == FLIP) {
+    const double flip = v0 + sa * A.dt;
+    *v = A.blending * flip + (1.0 - A.blending) * sv;
+  } else if (vu == ASFLIP) {  // particle.tcc:1097-1111
+    const double flip = v0 + sa * A.dt;
+    *v = A.blending * flip + (1.0 - A.blending) * sv;
+    *dx = beta * A.blending * flip + (1.0 - beta * A.blending) * sv;
+  } else {
+    *v = sv;
+  }
 }
 
 // Particle-level dN/dx at its xi.
@@ -846,6 +867,245 @@ __global__ __launch_bounds__(CH) void k_p2g(Mesh M, Particles P, Nodes Nd, StepA
   scatter_segments<D, WHAT, CH>(st, cnt, M, Nd, g);
 }
 
+// ----------------------- 3D fast mode: stress update -------------------------
+// Occupancy: 3 waves per SIMD for k_stress_fast on box cells (14 spilled
+// registers in the return mapping; collapse 345 us, slope 541 us, against 359
+// and 585 us at 2 waves without spills), 2 for the USF scatter (146 against
+// 160 us, 570k particles) and the general cells (92 against 132 us, 254k).
+// The stress update of a workgroup of BS particles (every thread calls it;
+// `live`: the thread has a particle p in a cell, its fields loaded and its
+// velocity gradient formed): kinematics, elastic predictor, and the return
+// mappings of the particles that yield, compacted over the workgroup in LDS.
+// KEEP: q.s is the new stress afterwards (through the LDS slots), else only
+// memory holds it.
+template <int D, bool KEEP, int BS>
+MPMX_DEV void block_stress_update(fast::Returns<BS>& R, bool live, const Particles& P,
+                                  const Material* mats, int p, fast::StressIn<D>& q,
+                                  const double (*L)[D], double div_c, double dt) {
+  const int64_t np = P.np;
+  const int tid = threadIdx.x;
+  if (tid < 2) R.n[tid] = 0;
+  __syncthreads();
+  int slot = -1;
+  if (live) {
+    const Material& m = mats[q.mat];
+    double sv[NSV];
+    if (m.type != LE) load_sv(P, m, p, sv);
+    double ds[6];
+    fast::strain_update<D>(P, p, q, L, div_c, dt, ds);
+    bool done = true;
+    if (m.type == LE) {
+      double t[6];
+      de_mul(m, ds, t);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) q.s[k] = q.s[k] + t[k];
+    } else {
+      int yt = FS_ELASTIC;
+      double y0 = 0.;
+      done = fast::predictor(m, q.s, ds, q.rho, sv, yt, y0);
+      if (done) {
+        store_sv(P, m, p, sv);
+      } else {  // the yield state and softened strength now, the rest below
+        stream_st(&P.sv[SV_YIELD * np + p], sv[SV_YIELD]);
+        if (m.softening) {
+          P.sv[SV_PHI * np + p] = sv[SV_PHI];
+          P.sv[SV_PSI * np + p] = sv[SV_PSI];
+          P.sv[SV_COH * np + p] = sv[SV_COH];
+          P.sv[SV_TCUT * np + p] = sv[SV_TCUT];
+        }
+        slot = fast::push_return<BS>(R, p, q.mat, q.s, ds, yt, y0);
+      }
+    }
+    if (done) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) stream_st(&P.stress[k * np + p], q.s[k]);
+    }
+  }
+  __syncthreads();
+  const int ns = R.n[0], nt = R.n[1];
+  if (tid < ns || tid >= BS - nt) {
+    const int pr = R.p[tid];
+    const Material& m = mats[R.mat[tid]];
+    double s[6], ds[6], sv[NSV];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      s[k] = R.s[k][tid];
+      ds[k] = R.ds[k][tid];
+    }
+    load_sv(P, m, pr, sv);
+    fast::plastic_return(m, s, ds, tid < ns ? FS_SHEAR : FS_TENSILE, R.y0[tid], sv);
+    stream_st(&P.sv[SV_EPS * np + pr], sv[SV_EPS]);
+    stream_st(&P.sv[SV_RHO * np + pr], sv[SV_RHO]);
+    stream_st(&P.sv[SV_THETA * np + pr], sv[SV_THETA]);
+    stream_st(&P.sv[SV_PDS * np + pr], sv[SV_PDS]);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      stream_st(&P.stress[k * np + pr], s[k]);
+      if constexpr (KEEP) R.s[k][tid] = s[k];
+    }
+  }
+  if constexpr (KEEP) {
+    __syncthreads();
+    if (slot >= 0) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) q.s[k] = R.s[k][slot];
+    }
+  }
+}
+
+// Velocity gradient of particle p's cell c from the nodes' velocities nv.
+template <int D, bool BOX>
+MPMX_DEV void velocity_gradient(const Mesh& M, int c, const double* xi, const double (*nv)[D],
+                                double (*L)[D], double* div_c) {
+  if constexpr (BOX) {
+    double len[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) len[k] = M.len[k * M.ncells + c];
+    fast::box_gradient<D>(xi, len, nv, L, div_c);
+  } else {
+    fast::cell_gradient<D>(M, c, xi, nv, L, div_c);
+  }
+}
+
+// Fast mode's k_stress (MUSL), particles in particle order.
+template <int D, bool BOX, bool LOCATE>
+__global__ __launch_bounds__(kStressBlock) MPMX_WAVES(BOX ? 3 : 2) void k_stress_fast(
+    Mesh M, Particles P, Nodes Nd, const Material* mats, StepArgs A, Status* S, int* scan_list) {
+  if (run_stopped(S)) return;
+  __shared__ fast::Returns<kStressBlock> R;
+  constexpr int NN = Elem<D>::NN;
+  const int64_t np = P.np;
+  const int64_t p = blockIdx.x * (int64_t)kStressBlock + threadIdx.x;
+  const int c = p < np ? P.cell[p] : -1;
+  const bool live = valid_cell<D>(M, c);
+  double L[D][D], div_c = 0., x[D];
+  fast::StressIn<D> q;
+  if (live) {
+    double xi[D], nv[NN][D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) xi[k] = P.xi[k * np + p];
+    gather_nodes<D>(M, Nd, c, nv, nullptr);
+    fast::load_stress_in<D>(P, p, q);
+    if constexpr (LOCATE) {
+#pragma unroll
+      for (int k = 0; k < D; ++k) x[k] = stream_ld(&P.x[k * np + p]);
+    }
+    velocity_gradient<D, BOX>(M, c, xi, nv, L, &div_c);
+    if constexpr (LOCATE) locate_one<D>(M, P, S, scan_list, (int)p, x, c, -1);
+  }
+  block_stress_update<D, false, kStressBlock>(R, live, P, mats, (int)p, q, L, div_c, A.dt);
+}
+
+// Fast mode's USF stress update in sorted order, then the force scatter of
+// the new stress.
+template <int D, bool BOX, int CH>
+__global__ __launch_bounds__(CH) MPMX_WAVES(2) void k_stress_scatter_fast(
+    Mesh M, Particles P, Nodes Nd, const Material* mats, StepArgs A, const Status* S,
+    const int* skey, const int* perm) {
+  if (run_stopped(S)) return;
+  constexpr int NN = Elem<D>::NN;
+  __shared__ union {
+    Stage<D, SC_F, CH> st;
+    fast::Returns<CH> R;
+  } sh;
+  const int64_t base = blockIdx.x * (int64_t)CH;
+  const int cnt = (int)((P.np - base) < CH ? (P.np - base) : CH);
+  const int tid = threadIdx.x;
+  const int64_t np = P.np;
+  const int key = tid < cnt ? skey[base + tid] : -1;
+  const int p = tid < cnt ? perm[base + tid] : 0;
+  const bool live = valid_cell<D>(M, key);
+  double xi[D], L[D][D], div_c = 0., mass = 0.;
+  fast::StressIn<D> q;
+  if (live) {
+    double nv[NN][D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) xi[k] = P.xi[k * np + p];
+    mass = P.mass[p];
+    gather_nodes<D>(M, Nd, key, nv, nullptr);
+    fast::load_stress_in<D>(P, p, q);
+    velocity_gradient<D, BOX>(M, key, xi, nv, L, &div_c);
+  }
+  block_stress_update<D, true, CH>(sh.R, live, P, mats, p, q, L, div_c, A.dt);
+  __syncthreads();
+  if (tid < cnt) sh.st.key[tid] = live ? key : -1;
+  if (live) {
+    double X[NN][D], Ji[D][D], Bm[D * D];
+    load_cell_X<D>(M, key, X);
+    jacobian_inverse<D>(xi, X, Ji);
+    force_matrix<D>(q.s, q.vol, Ji, Bm);
+    sh.st.m[tid] = mass;
+#pragma unroll
+    for (int k = 0; k < D; ++k) sh.st.xi[k][tid] = xi[k];
+#pragma unroll
+    for (int k = 0; k < D * D; ++k) sh.st.B[k][tid] = Bm[k];
+  }
+  double g[3] = {0, 0, 0};
+  gravity_now(A, S, D, g);
+  __syncthreads();
+  scatter_segments<D, SC_F, CH>(sh.st, cnt, M, Nd, g);
+}
+
+// Fast mode's k_g2p with the USL stress update.
+template <int D, bool BOX, bool LOCATE>
+__global__ __launch_bounds__(kBlock) MPMX_WAVES(2) void k_g2p_stress_fast(
+    Mesh M, Particles P, Nodes Nd, const Material* mats, StepArgs A, int vu, Status* S,
+    int* scan_list) {
+  if (run_stopped(S)) return;
+  __shared__ fast::Returns<kBlock> R;
+  constexpr int NN = Elem<D>::NN;
+  const int64_t np = P.np;
+  const int64_t p = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  const int c = p < np ? P.cell[p] : -1;
+  const bool live = valid_cell<D>(M, c);
+  double L[D][D], div_c = 0.;
+  fast::StressIn<D> q;
+  if (live) {
+    double xi[D], N[NN], nv[NN][D], sv[D], sa[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      xi[k] = P.xi[k * np + p];
+      sv[k] = sa[k] = 0.;
+    }
+    shapefn<D>(xi, N);
+    {
+#pragma clang fp contract(fast)
+      double na[NN][D];
+      gather_nodes<D>(M, Nd, c, nv, na);
+#pragma unroll
+      for (int i = 0; i < NN; ++i)
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+          sv[k] += N[i] * nv[i][k];
+          sa[k] += N[i] * na[i][k];
+        }
+    }
+    double x[D], v0[D], u0[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) {  // loads before stores (see kinematics)
+      v0[k] = stream_ld(&P.v[k * np + p]);
+      x[k] = stream_ld(&P.x[k * np + p]);
+      u0[k] = stream_ld(&P.u[k * np + p]);
+    }
+    fast::load_stress_in<D>(P, p, q);
+    const int pvc = P.pvc_mask ? P.pvc_mask[p] : 0;
+    const double beta = vu == ASFLIP ? P.beta[p] : 0.;
+    velocity_gradient<D, BOX>(M, c, xi, nv, L, &div_c);
+#pragma unroll
+    for (int k = 0; k < D; ++k) {
+      double v, dx;
+      update_velocity(vu, A, beta, v0[k], sv[k], sa[k], &v, &dx);
+      if (pvc & (1 << k)) v = P.pvc_val[k * np + p];  // particle.tcc:1190-1195
+      stream_st(&P.v[k * np + p], v);
+      x[k] = x[k] + dx * A.dt;
+      stream_st(&P.x[k * np + p], x[k]);
+      stream_st(&P.u[k * np + p], u0[k] + dx * A.dt);
+    }
+    if constexpr (LOCATE) locate_one<D>(M, P, S, scan_list, (int)p, x, c, -1);
+  }
+  block_stress_update<D, false, kBlock>(R, live, P, mats, (int)p, q, L, div_c, A.dt);
+}
+
 // USF stress update in sorted order, then the force scatter of the new stress.
 template <int D, int CH, bool ROT>
 __global__ __launch_bounds__(CH) MPMX_MC_ATTR void k_stress_scatter(Mesh M, Particles P, Nodes Nd,
@@ -961,18 +1221,8 @@ __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_g2p(Mesh M, Particles
   const double beta = vu == ASFLIP ? P.beta[p] : 0.;
 #pragma unroll
   for (int k = 0; k < D; ++k) {
-    double v = v0[k];
-    double dx = sv[k];  // position increment velocity
-    if (vu == FLIP) {
-      v += sa[k] * A.dt;
-      v = A.blending * v + (1.0 - A.blending) * sv[k];
-    } else if (vu == ASFLIP) {  // particle.tcc:1097-1111
-      const double flip = v + sa[k] * A.dt;
-      v = A.blending * flip + (1.0 - A.blending) * sv[k];
-      dx = beta * A.blending * flip + (1.0 - beta * A.blending) * sv[k];
-    } else {
-      v = sv[k];
-    }
+    double v, dx;
+    update_velocity(vu, A, beta, v0[k], sv[k], sa[k], &v, &dx);
     if (pvc & (1 << k)) v = P.pvc_val[k * np + p];  // particle.tcc:1190-1195
     stream_st(&P.v[k * np + p], v);
     x[k] = x[k] + dx * A.dt;
@@ -1932,21 +2182,43 @@ template <int D>
 void launch_stress_scatter(int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
                            const Material* mats, const StepArgs& A, const Status* S,
                            const int* skey, const int* perm, hipStream_t st) {
-#define L_(CH)                                                                                 \
-  if (P.spin)                                                                                  \
-    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, true>), P.np, st, M, P, Nd, mats, A, S, skey, \
-                   perm);                                                                      \
-  else                                                                                         \
-    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, false>), P.np, st, M, P, Nd, mats, A, S, skey, \
-                   perm)
+  // a stress rate (P.spin) runs the builds with the rotations
+#define L_(CH)                                                                                   \
+  if (P.spin)                                                                                    \
+    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, true>), P.np, st, M, P, Nd, mats, A, S, skey,   \
+                   perm);                                                                        \
+  else if constexpr (D == 2)                                                                     \
+    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, false>), P.np, st, M, P, Nd, mats, A, S, skey,  \
+                   perm);                                                                        \
+  else if (M.box)                                                                                \
+    MPMX_LAUNCH_CH(CH, (k_stress_scatter_fast<D, true, CH>), P.np, st, M, P, Nd, mats, A, S,    \
+                   skey, perm);                                                                  \
+  else                                                                                           \
+    MPMX_LAUNCH_CH(CH, (k_stress_scatter_fast<D, false, CH>), P.np, st, M, P, Nd, mats, A, S,   \
+                   skey, perm)
   MPMX_CHUNK_DISPATCH(chunk, L_);
 #undef L_
 }
 
 template <int D>
-void launch_stress(bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
+void launch_stress(bool fast, bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
                    const Material* mats, const StepArgs& A, Status* S, int* scan_list,
                    hipStream_t st) {
+  if constexpr (D == 3) if (fast) {
+    if (M.box && locate)
+      MPMX_LAUNCH_CH(kStressBlock, (k_stress_fast<D, true, true>), P.np, st, M, P, Nd, mats, A, S,
+                     scan_list);
+    else if (locate)
+      MPMX_LAUNCH_CH(kStressBlock, (k_stress_fast<D, false, true>), P.np, st, M, P, Nd, mats, A,
+                     S, scan_list);
+    else if (M.box)
+      MPMX_LAUNCH_CH(kStressBlock, (k_stress_fast<D, true, false>), P.np, st, M, P, Nd, mats, A,
+                     S, scan_list);
+    else
+      MPMX_LAUNCH_CH(kStressBlock, (k_stress_fast<D, false, false>), P.np, st, M, P, Nd, mats, A,
+                     S, scan_list);
+    return;
+  }
   // the Jaumann-rate build only when such a material exists (P.spin set)
   if (locate && P.spin)
     MPMX_LAUNCH_CH(kStressBlock, (k_stress<D, true, true>), P.np, st, M, P, Nd, mats, A, S,
@@ -1976,9 +2248,20 @@ void launch_plastic(const Particles& P, const Material* mats, const Status* S, h
 }
 
 template <int D>
-void launch_g2p(bool stress, bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
+void launch_g2p(bool fast, bool stress, bool locate, const Mesh& M, const Particles& P, const Nodes& Nd,
                 const Material* mats, const StepArgs& A, int vu, Status* S, int* scan_list,
                 hipStream_t st) {
+  if constexpr (D == 3) if (fast && stress) {
+    if (M.box && locate)
+      MPMX_LAUNCH((k_g2p_stress_fast<D, true, true>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
+    else if (locate)
+      MPMX_LAUNCH((k_g2p_stress_fast<D, false, true>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
+    else if (M.box)
+      MPMX_LAUNCH((k_g2p_stress_fast<D, true, false>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
+    else
+      MPMX_LAUNCH((k_g2p_stress_fast<D, false, false>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
+    return;
+  }
   if (stress && locate && P.spin)
     MPMX_LAUNCH((k_g2p<D, true, true, true>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
   else if (stress && locate)
@@ -2080,10 +2363,10 @@ template void take_rows<int>(const int*, int*, const int*, int64_t, int64_t, int
   template void launch_stress_scatter<D>(int, const Mesh&, const Particles&, const Nodes&,   \
                                          const Material*, const StepArgs&, const Status*,    \
                                          const int*, const int*, hipStream_t);               \
-  template void launch_stress<D>(bool, const Mesh&, const Particles&, const Nodes&,           \
+  template void launch_stress<D>(bool, bool, const Mesh&, const Particles&, const Nodes&,           \
                                  const Material*, const StepArgs&, Status*, int*,            \
                                  hipStream_t);                                               \
-  template void launch_g2p<D>(bool, bool, const Mesh&, const Particles&, const Nodes&,       \
+  template void launch_g2p<D>(bool, bool, bool, const Mesh&, const Particles&, const Nodes&,       \
                               const Material*, const StepArgs&, int, Status*, int*,          \
                               hipStream_t);                                                  \
   template void launch_g2p_scatter<D>(int, const Mesh&, const Particles&, const Nodes&,      \
