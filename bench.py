@@ -68,7 +68,7 @@ STEP_BYTES_PER_NODE = {3: 256, 2: 176}
 def summarize_trace(path, first, count, scale=None):
     """Per-kernel statistics of the dispatches in a rocprofv3 CSV (kernel
     trace, or one counter of a --pmc pass) that belong to simulated steps
-    first+1 .. first+count of the run: those after the first-th k_step_end
+    first+1 .. first+count of the run: those after the first-th k_step_tail
     dispatch up to the (first+count)-th. Steps are counted from the first
     solver the command creates, so run it without the autotuner (--chunk and
     --sort-every fixed), whose trial steps would shift the count. Returns
@@ -82,7 +82,7 @@ def summarize_trace(path, first, count, scale=None):
         name = r["Kernel_Name"]
         if first <= ends < first + count:
             sel.append(r)
-        if name.startswith("mpmx::k_step_end"):
+        if "mpmx::k_step_tail" in name:
             ends += 1
     if ends < first + count:
         raise SystemExit("only %d steps in %s" % (ends, path))

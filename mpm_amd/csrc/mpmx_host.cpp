@@ -179,23 +179,28 @@ struct mpmx_ctx {
   DBuf<double> d_plastic_rec;
   DBuf<Status> d_status;
   Status* h_status = nullptr;  // pinned
+  // the device's status block is what reset_status would write for step
+  // status_step (but for ad_slot): the last run ended without a lost particle
+  bool status_clean = false;
+  bool published = false;  // the queued run leaves its status in h_status itself
+  int64_t status_step = 0;
   double g[3] = {0, 0, 0};
   double ramp = 0;
   int64_t step = 0;
 
   // particle order by cell: a full radix sort every `sort_every` steps (and
   // whenever the particle set changed); in between, fast mode reuses the last
-  // permutation with refreshed keys
+  // permutation (the scatter kernels read the particles' current cells)
   int sort_every = 8;
   int chunk = 256;  // particles per workgroup of the LDS-staged scatters
   bool need_sort = true;
   int64_t since_sort = 0;
 
-  // graph cache: [0] step with key refresh, [1] step with a full sort
-  // [2], [3]: the same steps recording nodal quantities into the slots of
-  // d_ad_node_slots (the slot index is Status::ad_slot)
-  hipGraphExec_t graph_exec[4] = {nullptr, nullptr, nullptr, nullptr};
+  // graph cache: blocks of kBlockSteps steps, [0] in the last sort's order,
+  // [1] the first of them with a full sort (ordered mode: all of them)
+  hipGraphExec_t graph_exec[2] = {};
   double graph_dt = 0, graph_damping = 0;
+  int64_t graph_steps = 0;  // steps queued since the graphs were invalidated
 
   // adjoint: checkpoints of a recorded run (full particle state every
   // ad_every steps and at its end), the per-step records of one segment, node
@@ -240,6 +245,7 @@ struct mpmx_ctx {
       if (g) (void)hipGraphExecDestroy(g);
       g = nullptr;
     }
+    graph_steps = 0;
   }
 
   Mesh mesh() const {
@@ -832,13 +838,16 @@ void reset_status(mpmx_ctx* c) {
   s.nplastic = 0;
   s.nplastic_t = 0;
   s.ad_slot = 0;
+  s.ticket = 0;
   s.nlost = 0;
+  c->status_clean = c->published = false;
   *c->h_status = s;
   c->d_status.upload(c->h_status, 1, c->stream);
 }
 
 void read_status(mpmx_ctx* c) {
-  c->d_status.download(c->h_status, 1, c->stream);
+  if (!c->published) c->d_status.download(c->h_status, 1, c->stream);
+  c->published = false;
   HIPCHECK(hipStreamSynchronize(c->stream));
 }
 
@@ -1012,6 +1021,7 @@ struct StepBuffers {
   double* rotF;   // Green-Naghdi scratch; rotated trial stresses of the deferred list
   double* plastic_trial;
   double* gterm;  // ordered mode: per-particle gather terms
+  Status* host = nullptr;  // pinned memory that takes the status at the step's end
 };
 
 StepBuffers ctx_buffers(mpmx_ctx* c) {
@@ -1137,8 +1147,6 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
     L("sort_by_cell", [&] {
       radix_sort_by_cell(P.cell, P.np, (int)M.ncells, skey, perm, B.sort_tmp, st);
     });
-  else
-    L("refresh_keys", [&] { refresh_sorted_keys(P.cell, perm, P.np, (int)M.ncells, skey, st); });
   if (ordered) {
     L("cell_ranges", [&] {
       launch_cell_ranges<D>(P.np, M.ncells, skey, B.cstart, B.cend, st);
@@ -1170,31 +1178,31 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
   } else {
     affine();
     if (c->scheme == USF) {
-      L("p2g_mass_momentum", [&] { launch_p2g<D>(P2G_MV, c->chunk, M, P, Nd, A, S, skey, perm, st); });
+      L("p2g_mass_momentum", [&] { launch_p2g<D>(P2G_MV, c->chunk, M, P, Nd, A, S, perm, st); });
       L("node_velocity", [&] { launch_node<D>(ND_INIT | ND_VEL, M, Nd, A, S, st); });
-      L("stress_force_scatter", [&] { launch_stress_scatter<D>(c->chunk, M, P, Nd, mats, A, S, skey, perm, st); });
+      L("stress_force_scatter", [&] { launch_stress_scatter<D>(c->chunk, M, P, Nd, mats, A, S, perm, st); });
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_acceleration", [&] { launch_node<D>(ND_ACC | ND_ZERO_ALL, M, Nd, A, S, st); });
       mapping();
       L("g2p_locate", [&] { launch_g2p<D>(own, false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
     } else if (c->scheme == USL) {
-      L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, skey, perm, st); });
+      L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, perm, st); });
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_update", [&] { launch_node<D>(ND_INIT | ND_VEL | ND_ACC | ND_ZERO_ALL, M, Nd, A, S, st); });
       mapping();
       L("g2p_stress_locate", [&] { launch_g2p<D>(own, true, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
       plastic();
     } else {
-      L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, skey, perm, st); });
+      L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, perm, st); });
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_update", [&] { launch_node<D>(ND_INIT | ND_VEL | ND_ACC | ND_ZERO_MOM, M, Nd, A, S, st); });
       if (aff) {  // G2P, then the affine momentum map with the new positions
         mapping();
         L("g2p", [&] { launch_g2p<D>(own, false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
         affine();
-        L("p2g_momentum", [&] { launch_p2g<D>(P2G_MOM, c->chunk, M, P, Nd, A, S, skey, perm, st); });
+        L("p2g_momentum", [&] { launch_p2g<D>(P2G_MOM, c->chunk, M, P, Nd, A, S, perm, st); });
       } else {
-        L("g2p_momentum_scatter", [&] { launch_g2p_scatter<D>(c->chunk, M, P, Nd, A, c->vu, S, skey, perm, st); });
+        L("g2p_momentum_scatter", [&] { launch_g2p_scatter<D>(c->chunk, M, P, Nd, A, c->vu, S, perm, st); });
       }
       L("node_velocity", [&] { launch_node<D>(ND_VEL | ND_ZERO_ALL, M, Nd, A, S, st); });
       L("stress_locate", [&] { launch_stress<D>(own, loc, M, P, Nd, mats, A, S, scan, st); });
@@ -1202,8 +1210,13 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
     }
   }
   if (!loc) L("locate", [&] { launch_locate_step<D>(!ordered, M, P, S, scan, st); });
-  L("locate_scan", [&] { launch_locate_scan<D>(M, P, S, scan, nullptr, c->locate_all ? 0 : 1, st); });
-  L("step_end", [&] { launch_step_end(S, st); });
+  const int remove_lost = c->locate_all ? 0 : 1;
+  if (c->profile) {  // timed apart
+    L("locate_scan", [&] { launch_locate_scan<D>(M, P, S, scan, nullptr, remove_lost, st); });
+    L("step_end", [&] { launch_step_end(S, st); });
+  } else {
+    launch_step_tail<D>(M, P, S, scan, remove_lost, B.host, st);
+  }
 }
 
 void enqueue(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
@@ -1224,9 +1237,6 @@ bool next_step_sorts(mpmx_ctx* c) {
 }
 
 
-// Queue nsteps steps on the context's stream (one graph replay each).
-// ad_nodes: record each step's nodal quantities in the slots of length
-// ad_stride there, step Status::ad_slot in its slot.
 StepArgs step_args(const mpmx_ctx* c, double dt, double damping) {
   StepArgs A;
   A.dt = dt;
@@ -1241,6 +1251,18 @@ StepArgs step_args(const mpmx_ctx* c, double dt, double damping) {
   return A;
 }
 
+// Steps per graph. A graph of one step is slower than launching its kernels
+// (8 us idle between two graph launches; a single step's call 45.6 against
+// 39.6 us, 512 particles); of four it is faster (20 steps 528 against 558 us),
+// and a sort interval holds at least one such block.
+constexpr int kBlockSteps = 4;
+// Steps launched directly before the first capture: capturing and
+// instantiating costs some 300 us, more than a short run gains.
+constexpr int64_t kGraphAfter = 24;
+
+// Queue nsteps steps on the context's stream. ad_nodes: record each step's
+// nodal quantities in the slots of length ad_stride there, step
+// Status::ad_slot in its slot.
 void launch_steps(mpmx_ctx* c, int nsteps, double dt, double damping,
                   double* ad_nodes = nullptr, int64_t ad_stride = 0, int ad_nslots = 0) {
   const StepBuffers B = ctx_buffers(c);
@@ -1255,33 +1277,48 @@ void launch_steps(mpmx_ctx* c, int nsteps, double dt, double damping,
   A.ad_stride = ad_stride;
   A.ad_nslots = ad_nslots;
   Launcher L{c};
-  const bool use_graph = !(c->flags & MPMX_NO_GRAPH) && !c->profile;
-  const int rec = ad_nodes ? 2 : 0;
-  if (use_graph) {
-    if (c->graph_dt != dt || c->graph_damping != damping) {
-      c->invalidate_graph();
-      c->graph_dt = dt;
-      c->graph_damping = damping;
-    }
-    for (int s = 0; s < nsteps; ++s) {
-      const int kind = (next_step_sorts(c) ? 1 : 0) + rec;
-      if (!c->graph_exec[kind]) {
+  // recorded steps come one by one: launched directly
+  const bool use_graph = !(c->flags & MPMX_NO_GRAPH) && !c->profile && !ad_nodes;
+  if (c->graph_dt != dt || c->graph_damping != damping) {
+    c->invalidate_graph();
+    c->graph_dt = dt;
+    c->graph_damping = damping;
+  }
+  const bool ordered = (c->flags & MPMX_ORDERED) != 0;
+  c->published = false;
+  for (int s = 0; s < nsteps;) {
+    const bool sorts = ordered || c->need_sort || c->since_sort >= c->sort_every;
+    // steps until the next sort (ordered mode sorts in every step)
+    const int64_t run = ordered ? nsteps : (sorts ? c->sort_every : c->sort_every - c->since_sort);
+    if (use_graph && c->graph_steps >= kGraphAfter &&
+        std::min<int64_t>(run, nsteps - s) >= kBlockSteps) {
+      hipGraphExec_t& exec = c->graph_exec[sorts ? 1 : 0];
+      if (!exec) {
         hipGraph_t graph;
         HIPCHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        enqueue(c, A, L, (kind & 1) == 1, B);
+        for (int k = 0; k < kBlockSteps; ++k) enqueue(c, A, L, sorts && (ordered || k == 0), B);
         HIPCHECK(hipStreamEndCapture(c->stream, &graph));
-        hipError_t e = hipGraphInstantiate(&c->graph_exec[kind], graph, nullptr, nullptr, 0);
+        hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         HIPCHECK(e);
       }
-      HIPCHECK(hipGraphLaunch(c->graph_exec[kind], c->stream));
+      HIPCHECK(hipGraphLaunch(exec, c->stream));
+      for (int k = 0; k < kBlockSteps; ++k) (void)next_step_sorts(c);
+      c->graph_steps += kBlockSteps;
+      s += kBlockSteps;
+      continue;
     }
-  } else {
-    for (int s = 0; s < nsteps; ++s) {
-      enqueue(c, A, L, next_step_sorts(c), B);
-      HIPCHECK(hipGetLastError());
-      L.collect();
+    // the last step of a call also leaves the status in pinned host memory
+    StepBuffers Bs = B;
+    if (s == nsteps - 1 && !c->profile && !ad_nodes) {
+      Bs.host = c->h_status;
+      c->published = true;
     }
+    enqueue(c, A, L, next_step_sorts(c), Bs);
+    HIPCHECK(hipGetLastError());
+    L.collect();
+    ++c->graph_steps;
+    ++s;
   }
 }
 
@@ -1357,6 +1394,9 @@ void remove_lost_particles(mpmx_ctx* c) {
 void check_status(mpmx_ctx* c) {
   read_status(c);
   c->step = c->h_status->step;
+  c->status_clean = c->h_status->nlost == 0 &&
+                    c->h_status->first_bad_step == std::numeric_limits<int64_t>::max();
+  c->status_step = c->step;
   if (c->h_status->nlost > 0) remove_lost_particles(c);
   if (c->h_status->first_bad_step != std::numeric_limits<int64_t>::max())
     throw ApiError(MPMX_E_UNLOCATABLE,
@@ -1505,16 +1545,10 @@ void ad_save_slot(mpmx_ctx* c, int j) {
 // second momentum and its velocity.
 int64_t ad_node_slot_doubles(const mpmx_ctx* c) { return (1 + 6 * c->dim) * c->nnodes; }
 // The step records of one segment: K + 1 particle slots and K nodal slots.
-// The recording graphs hold their addresses, so they are captured anew.
 void ad_alloc_slots(mpmx_ctx* c, int K) {
   c->d_ad_slots.alloc((size_t)(K + 1) * ad_slot_doubles(c));
   c->d_ad_slot_cell.alloc((size_t)(K + 1) * c->np);
   c->d_ad_node_slots.alloc((size_t)K * ad_node_slot_doubles(c));
-  for (int k = 2; k < 4; ++k)
-    if (c->graph_exec[k]) {
-      (void)hipGraphExecDestroy(c->graph_exec[k]);
-      c->graph_exec[k] = nullptr;
-    }
 }
 
 double* ad_node_slot(mpmx_ctx* c, int j) {
@@ -2330,7 +2364,8 @@ int mpmx_step(mpmx_ctx* c, int nsteps, double dt, double damping_factor) {
     c->step += nsteps;
     return MPMX_OK;
   }
-  reset_status(c);
+  if (!c->status_clean || c->status_step != c->step) reset_status(c);
+  c->status_clean = false;  // until the run has ended well
   launch_steps(c, nsteps, dt, damping_factor);
   check_status(c);
   API_END(c)
@@ -2716,8 +2751,11 @@ int mpmx_adjoint_backward_device(mpmx_ctx* c, const double* dL_dx, const double*
 int mpmx_get_particles_device(mpmx_ctx* c, double* x, double* v) {
   API_BEGIN(c)
   if (c->np == 0) return MPMX_OK;
-  if (x) launch_soa_to_rows(c->d_x.p, x, c->np, c->dim, 1.0, nullptr, nullptr, nullptr, c->stream);
-  if (v) launch_soa_to_rows(c->d_v.p, v, c->np, c->dim, 1.0, nullptr, nullptr, nullptr, c->stream);
+  if (!x && !v) return MPMX_OK;
+  if (c->dim == 2)
+    launch_rows_xv<2>(c->parts(), x, v, c->stream);
+  else
+    launch_rows_xv<3>(c->parts(), x, v, c->stream);
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipStreamSynchronize(c->stream));
   API_END(c)
@@ -2740,11 +2778,6 @@ int mpmx_adjoint_release(mpmx_ctx* c) {
   c->d_ad_slots.release();
   c->d_ad_slot_cell.release();
   c->d_ad_node_slots.release();
-  for (int k = 2; k < 4; ++k)
-    if (c->graph_exec[k]) {
-      (void)hipGraphExecDestroy(c->graph_exec[k]);
-      c->graph_exec[k] = nullptr;
-    }
   c->d_ad_nodes.release();
   c->d_ad_parts.release();
   c->d_ad_list.release();

@@ -38,6 +38,11 @@ template <int D>
 void launch_locate_scan(const Mesh& M, const Particles& P, Status* S, const int* scan_list,
                         const int* hint, int remove_lost, hipStream_t st);
 void launch_step_end(Status* S, hipStream_t st);
+// launch_locate_scan of a step and launch_step_end in one kernel; host: pinned
+// memory that takes the status block, or null
+template <int D>
+void launch_step_tail(const Mesh& M, const Particles& P, Status* S, const int* scan_list,
+                      int remove_lost, Status* host, hipStream_t st);
 // values of the nf (<= kMaxMathFns) math functions at the current step's time
 constexpr int kMaxMathFns = 256;
 void launch_fn_eval(const MathFn* fns, const double* data, int nf, const Status* S, double dt,
@@ -45,12 +50,11 @@ void launch_fn_eval(const MathFn* fns, const double* data, int nf, const Status*
 // chunk: particles per workgroup of the LDS-staged scatters (128, 256, 512)
 template <int D>
 void launch_p2g(int what, int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
-                const StepArgs& A, const Status* S, const int* skey, const int* perm,
-                hipStream_t st);
+                const StepArgs& A, const Status* S, const int* perm, hipStream_t st);
 template <int D>
 void launch_stress_scatter(int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
                            const Material* mats, const StepArgs& A, const Status* S,
-                           const int* skey, const int* perm, hipStream_t st);
+                           const int* perm, hipStream_t st);
 // fast: fast mode without a stress rate; the kernels then complete their own
 // return mappings (launch_plastic is not needed).
 template <int D>
@@ -71,8 +75,8 @@ void launch_g2p(bool fast, bool stress, bool locate, const Mesh& M, const Partic
                 hipStream_t st);
 template <int D>
 void launch_g2p_scatter(int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
-                        const StepArgs& A, int vu, const Status* S, const int* skey,
-                        const int* perm, hipStream_t st);
+                        const StepArgs& A, int vu, const Status* S, const int* perm,
+                        hipStream_t st);
 template <int D>
 void launch_node(int fl, const Mesh& M, const Nodes& Nd, const StepArgs& A, const Status* S,
                  hipStream_t st);
@@ -83,6 +87,10 @@ template <int D>
 void launch_gather(int which, const Mesh& M, const Particles& P, const Nodes& Nd,
                    const StepArgs& A, const Status* S, const int* perm, const int* cstart,
                    const int* cend, hipStream_t st);
+
+// Positions and velocities as rows of D (either null).
+template <int D>
+void launch_rows_xv(const Particles& P, double* rx, double* rv, hipStream_t st);
 
 // out[k * nnew + i] = in[k * nold + idx[i]] for the comps components of a
 // component-major array (T = double or int).
@@ -97,9 +105,4 @@ void take_rows(const T* in, T* out, const int* idx, int64_t nnew, int64_t nold, 
 int64_t radix_sort_temp_ints(int64_t n);
 void radix_sort_by_cell(const int* cell, int64_t n, int max_key, int* keys_out, int* vals_out,
                         int* tmp, hipStream_t st);
-// keys[i] = cell[perm[i]] for an earlier sort's permutation (cells changed
-// since then leave the keys only nearly sorted).
-void refresh_sorted_keys(const int* cell, const int* perm, int64_t n, int max_key, int* keys,
-                         hipStream_t st);
-
 }  // namespace mpmx

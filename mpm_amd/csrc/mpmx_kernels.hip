@@ -486,12 +486,9 @@ __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_locate_step(Mesh M, P
 // stops the run (the reference throws, mpm_scheme.tcc:250-256) or, with
 // remove_lost, is counted for removal (mpm_scheme.tcc:258-260).
 template <int D>
-__global__ __launch_bounds__(kBlock) void k_locate_scan(Mesh M, Particles P, Status* S,
-                                                        const int* scan_list, const int* hint,
-                                                        int remove_lost) {
-  if (run_stopped(S)) return;
+MPMX_DEV void scan_queue(const Mesh& M, const Particles& P, Status* S, const int* scan_list,
+                         const int* hint, int remove_lost, int n) {
   __shared__ int best;
-  const int n = S->nscan;
   for (int q = blockIdx.x; q < n; q += gridDim.x) {
     const int p = scan_list[q];
     double x[D];
@@ -544,6 +541,14 @@ __global__ __launch_bounds__(kBlock) void k_locate_scan(Mesh M, Particles P, Sta
   }
 }
 
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_locate_scan(Mesh M, Particles P, Status* S,
+                                                        const int* scan_list, const int* hint,
+                                                        int remove_lost) {
+  if (run_stopped(S)) return;
+  scan_queue<D>(M, P, S, scan_list, hint, remove_lost, S->nscan);
+}
+
 // End of step: advance the counter, clear the scan queue.
 // Mesh::update_nodal_acceleration_constraints (mesh.tcc:1414-1428): the math
 // functions' values at current_time = step * dt (mpm_scheme.tcc:219).
@@ -553,14 +558,60 @@ __global__ void k_fn_eval(const MathFn* fns, const double* data, int nf, const S
   if (f < nf) out[f] = math_fn_value(fns[f], data, static_cast<double>(S->step) * dt);
 }
 
+MPMX_DEV void end_step(Status* S) {
+  S->step += 1;
+  S->nscan = 0;
+  S->nplastic = 0;
+  S->nplastic_t = 0;
+  S->ad_slot += 1;
+}
+
 __global__ void k_step_end(Status* S) {
   if (run_stopped(S)) return;
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    S->step += 1;
-    S->nscan = 0;
-    S->nplastic = 0;
-    S->nplastic_t = 0;
-    S->ad_slot += 1;
+  if (threadIdx.x == 0 && blockIdx.x == 0) end_step(S);
+}
+
+// The scan of queued particles and the end of the step in one launch (a
+// launch costs 4 us whatever it does, and the queue is empty in almost every
+// step). Empty queue: one thread ends the step; the other workgroups read only
+// the queue's length, which stays 0. Otherwise every workgroup scans its share
+// and the last one to finish, by a ticket, ends the step. `host`: pinned host
+// memory that takes the status block too (the last step of a call, which then
+// needs no copy), or null.
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_step_tail(Mesh M, Particles P, Status* S,
+                                                      const int* scan_list, int remove_lost,
+                                                      Status* host) {
+  if (run_stopped(S)) {  // the state stays as the failed step left it
+    if (host && threadIdx.x == 0 && blockIdx.x == 0) *host = *S;
+    return;
+  }
+  const int n = S->nscan;
+  if (n == 0) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+      end_step(S);
+      if (host) *host = *S;
+    }
+    return;
+  }
+  scan_queue<D>(M, P, S, scan_list, nullptr, remove_lost, n);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    if (atomicAdd(&S->ticket, 1) == (int)gridDim.x - 1) {
+      S->ticket = 0;
+      end_step(S);
+      if (host) {  // what other workgroups changed, past this one's caches
+        Status h = *S;
+        h.first_bad_step =
+            __hip_atomic_load(&S->first_bad_step, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        h.bad_particle =
+            __hip_atomic_load(&S->bad_particle, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        h.nlost = __hip_atomic_load(&S->nlost, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        h.ticket = 0;
+        *host = h;
+      }
+    }
   }
 }
 
@@ -818,8 +869,7 @@ MPMX_DEV void gravity_now(const StepArgs& A, const Status* S, int dim, double* g
 // mpm_scheme.tcc:44-71 and 131-190; particle.tcc:630-658, 893-950.
 template <int D, int WHAT, int CH>
 __global__ __launch_bounds__(CH) void k_p2g(Mesh M, Particles P, Nodes Nd, StepArgs A,
-                                                const Status* S, const int* skey,
-                                                const int* perm) {
+                                                const Status* S, const int* perm) {
   if (run_stopped(S)) return;
   __shared__ Stage<D, WHAT, CH> st;
   const int64_t base = blockIdx.x * (int64_t)CH;
@@ -827,8 +877,8 @@ __global__ __launch_bounds__(CH) void k_p2g(Mesh M, Particles P, Nodes Nd, StepA
   const int tid = threadIdx.x;
   const int64_t np = P.np;
   if (tid < cnt) {
-    const int key = skey[base + tid];
     const int p = perm[base + tid];
+    const int key = P.cell[p];
     const bool ok = valid_cell<D>(M, key);
     st.key[tid] = ok ? key : -1;
     if (ok) {
@@ -1001,7 +1051,7 @@ __global__ __launch_bounds__(kStressBlock) MPMX_WAVES(BOX ? 3 : 2) void k_stress
 template <int D, bool BOX, int CH>
 __global__ __launch_bounds__(CH) MPMX_WAVES(2) void k_stress_scatter_fast(
     Mesh M, Particles P, Nodes Nd, const Material* mats, StepArgs A, const Status* S,
-    const int* skey, const int* perm) {
+    const int* perm) {
   if (run_stopped(S)) return;
   constexpr int NN = Elem<D>::NN;
   __shared__ union {
@@ -1012,8 +1062,8 @@ __global__ __launch_bounds__(CH) MPMX_WAVES(2) void k_stress_scatter_fast(
   const int cnt = (int)((P.np - base) < CH ? (P.np - base) : CH);
   const int tid = threadIdx.x;
   const int64_t np = P.np;
-  const int key = tid < cnt ? skey[base + tid] : -1;
   const int p = tid < cnt ? perm[base + tid] : 0;
+  const int key = tid < cnt ? P.cell[p] : -1;
   const bool live = valid_cell<D>(M, key);
   double xi[D], L[D][D], div_c = 0., mass = 0.;
   fast::StressIn<D> q;
@@ -1110,8 +1160,7 @@ __global__ __launch_bounds__(kBlock) MPMX_WAVES(2) void k_g2p_stress_fast(
 template <int D, int CH, bool ROT>
 __global__ __launch_bounds__(CH) MPMX_MC_ATTR void k_stress_scatter(Mesh M, Particles P, Nodes Nd,
                                                            const Material* mats, StepArgs A,
-                                                           const Status* S, const int* skey,
-                                                           const int* perm) {
+                                                           const Status* S, const int* perm) {
   if (run_stopped(S)) return;
   constexpr int NN = Elem<D>::NN;
   __shared__ Stage<D, SC_F, CH> st;
@@ -1120,8 +1169,8 @@ __global__ __launch_bounds__(CH) MPMX_MC_ATTR void k_stress_scatter(Mesh M, Part
   const int tid = threadIdx.x;
   const int64_t np = P.np;
   if (tid < cnt) {
-    const int key = skey[base + tid];
     const int p = perm[base + tid];
+    const int key = P.cell[p];
     const bool ok = valid_cell<D>(M, key);
     st.key[tid] = ok ? key : -1;
     if (ok) {
@@ -1454,7 +1503,7 @@ __global__ __launch_bounds__(kPlasticBlock) MPMX_PLASTIC_ATTR void k_plastic(Par
 // because the shape functions are not recomputed).
 template <int D, int CH>
 __global__ __launch_bounds__(CH) void k_g2p_scatter(Mesh M, Particles P, Nodes Nd, StepArgs A,
-                                                        int vu, const Status* S, const int* skey,
+                                                        int vu, const Status* S,
                                                         const int* perm) {
   if (run_stopped(S)) return;
   constexpr int NN = Elem<D>::NN;
@@ -1464,8 +1513,8 @@ __global__ __launch_bounds__(CH) void k_g2p_scatter(Mesh M, Particles P, Nodes N
   const int tid = threadIdx.x;
   const int64_t np = P.np;
   if (tid < cnt) {
-    const int key = skey[base + tid];
     const int p = perm[base + tid];
+    const int key = P.cell[p];
     const bool ok = valid_cell<D>(M, key);
     st.key[tid] = ok ? key : -1;
     if (ok) {
@@ -2142,6 +2191,13 @@ void launch_locate_scan(const Mesh& M, const Particles& P, Status* S, const int*
                      hint, remove_lost);
 }
 
+template <int D>
+void launch_step_tail(const Mesh& M, const Particles& P, Status* S, const int* scan_list,
+                      int remove_lost, Status* host, hipStream_t st) {
+  hipLaunchKernelGGL((k_step_tail<D>), dim3(256), dim3(kBlock), 0, st, M, P, S, scan_list,
+                     remove_lost, host);
+}
+
 void launch_fn_eval(const MathFn* fns, const double* data, int nf, const Status* S, double dt,
                     double* out, hipStream_t st) {
   if (nf <= 0) return;
@@ -2154,25 +2210,25 @@ void launch_step_end(Status* S, hipStream_t st) {
 
 template <int D>
 void launch_p2g(int what, int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
-                const StepArgs& A, const Status* S, const int* skey, const int* perm,
+                const StepArgs& A, const Status* S, const int* perm,
                 hipStream_t st) {
   if (P.Cmat) {  // affine velocity updates: 128-particle chunks
     if (what == SC_MV)
-      MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MV | SC_AFF, 128>), P.np, st, M, P, Nd, A, S, skey, perm);
+      MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MV | SC_AFF, 128>), P.np, st, M, P, Nd, A, S, perm);
     else if (what == SC_MOM)
-      MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MOM | SC_AFF, 128>), P.np, st, M, P, Nd, A, S, skey, perm);
+      MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MOM | SC_AFF, 128>), P.np, st, M, P, Nd, A, S, perm);
     else
-      MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MV | SC_F | SC_AFF, 128>), P.np, st, M, P, Nd, A, S, skey,
+      MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MV | SC_F | SC_AFF, 128>), P.np, st, M, P, Nd, A, S,
                      perm);
     return;
   }
   if (what == SC_MV) {
-#define L_(CH) MPMX_LAUNCH_CH(CH, (k_p2g<D, SC_MV, CH>), P.np, st, M, P, Nd, A, S, skey, perm)
+#define L_(CH) MPMX_LAUNCH_CH(CH, (k_p2g<D, SC_MV, CH>), P.np, st, M, P, Nd, A, S, perm)
     MPMX_CHUNK_DISPATCH(chunk, L_);
 #undef L_
   } else {
 #define L_(CH) \
-  MPMX_LAUNCH_CH(CH, (k_p2g<D, SC_MV | SC_F, CH>), P.np, st, M, P, Nd, A, S, skey, perm)
+  MPMX_LAUNCH_CH(CH, (k_p2g<D, SC_MV | SC_F, CH>), P.np, st, M, P, Nd, A, S, perm)
     MPMX_CHUNK_DISPATCH(chunk, L_);
 #undef L_
   }
@@ -2181,21 +2237,21 @@ void launch_p2g(int what, int chunk, const Mesh& M, const Particles& P, const No
 template <int D>
 void launch_stress_scatter(int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
                            const Material* mats, const StepArgs& A, const Status* S,
-                           const int* skey, const int* perm, hipStream_t st) {
+                           const int* perm, hipStream_t st) {
   // a stress rate (P.spin) runs the builds with the rotations
 #define L_(CH)                                                                                   \
   if (P.spin)                                                                                    \
-    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, true>), P.np, st, M, P, Nd, mats, A, S, skey,   \
+    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, true>), P.np, st, M, P, Nd, mats, A, S,   \
                    perm);                                                                        \
   else if constexpr (D == 2)                                                                     \
-    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, false>), P.np, st, M, P, Nd, mats, A, S, skey,  \
+    MPMX_LAUNCH_CH(CH, (k_stress_scatter<D, CH, false>), P.np, st, M, P, Nd, mats, A, S,  \
                    perm);                                                                        \
   else if (M.box)                                                                                \
     MPMX_LAUNCH_CH(CH, (k_stress_scatter_fast<D, true, CH>), P.np, st, M, P, Nd, mats, A, S,    \
-                   skey, perm);                                                                  \
+                   perm);                                                                  \
   else                                                                                           \
     MPMX_LAUNCH_CH(CH, (k_stress_scatter_fast<D, false, CH>), P.np, st, M, P, Nd, mats, A, S,   \
-                   skey, perm)
+                   perm)
   MPMX_CHUNK_DISPATCH(chunk, L_);
 #undef L_
 }
@@ -2278,9 +2334,9 @@ void launch_g2p(bool fast, bool stress, bool locate, const Mesh& M, const Partic
 
 template <int D>
 void launch_g2p_scatter(int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
-                        const StepArgs& A, int vu, const Status* S, const int* skey,
-                        const int* perm, hipStream_t st) {
-#define L_(CH) MPMX_LAUNCH_CH(CH, (k_g2p_scatter<D, CH>), P.np, st, M, P, Nd, A, vu, S, skey, perm)
+                        const StepArgs& A, int vu, const Status* S, const int* perm,
+                        hipStream_t st) {
+#define L_(CH) MPMX_LAUNCH_CH(CH, (k_g2p_scatter<D, CH>), P.np, st, M, P, Nd, A, vu, S, perm)
   MPMX_CHUNK_DISPATCH(chunk, L_);
 #undef L_
 }
@@ -2337,6 +2393,23 @@ void launch_gather(int which, const Mesh& M, const Particles& P, const Nodes& Nd
   }
 }
 
+// Positions and velocities as rows of D, either null.
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_rows_xv(const double* x, const double* v, double* rx,
+                                                    double* rv, int64_t n) {
+  const int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (i >= n) return;
+#pragma unroll
+  for (int k = 0; k < D; ++k) {
+    if (rx) rx[i * D + k] = x[k * n + i];
+    if (rv) rv[i * D + k] = v[k * n + i];
+  }
+}
+template <int D>
+void launch_rows_xv(const Particles& P, double* rx, double* rv, hipStream_t st) {
+  MPMX_LAUNCH((k_rows_xv<D>), P.np, st, P.x, P.v, rx, rv, P.np);
+}
+
 template <class T>
 void take_rows(const T* in, T* out, const int* idx, int64_t nnew, int64_t nold, int comps,
                hipStream_t st) {
@@ -2351,6 +2424,9 @@ template void take_rows<int>(const int*, int*, const int*, int64_t, int64_t, int
                                       const int*, hipStream_t);                              \
   template void launch_locate_scan<D>(const Mesh&, const Particles&, Status*, const int*,    \
                                       const int*, int, hipStream_t);                         \
+  template void launch_rows_xv<D>(const Particles&, double*, double*, hipStream_t);          \
+  template void launch_step_tail<D>(const Mesh&, const Particles&, Status*, const int*, int, \
+                                    Status*, hipStream_t);                                   \
   template void launch_locate_step<D>(bool, const Mesh&, const Particles&, Status*, int*,    \
                                       hipStream_t);                                          \
   template void launch_mapping_matrix<D>(const Mesh&, const Particles&, const Nodes&,        \
@@ -2358,11 +2434,10 @@ template void take_rows<int>(const int*, int*, const int*, int64_t, int64_t, int
   template void launch_affine_matrix<D>(const Mesh&, const Particles&, int, const Status*,   \
                                         hipStream_t);                                        \
   template void launch_p2g<D>(int, int, const Mesh&, const Particles&, const Nodes&,         \
-                              const StepArgs&, const Status*, const int*, const int*,        \
-                              hipStream_t);                                                  \
+                              const StepArgs&, const Status*, const int*, hipStream_t);      \
   template void launch_stress_scatter<D>(int, const Mesh&, const Particles&, const Nodes&,   \
                                          const Material*, const StepArgs&, const Status*,    \
-                                         const int*, const int*, hipStream_t);               \
+                                         const int*, hipStream_t);                           \
   template void launch_stress<D>(bool, bool, const Mesh&, const Particles&, const Nodes&,           \
                                  const Material*, const StepArgs&, Status*, int*,            \
                                  hipStream_t);                                               \
@@ -2371,7 +2446,7 @@ template void take_rows<int>(const int*, int*, const int*, int64_t, int64_t, int
                               hipStream_t);                                                  \
   template void launch_g2p_scatter<D>(int, const Mesh&, const Particles&, const Nodes&,      \
                                       const StepArgs&, int, const Status*, const int*,       \
-                                      const int*, hipStream_t);                              \
+                                      hipStream_t);                                          \
   template void launch_node<D>(int, const Mesh&, const Nodes&, const StepArgs&,             \
                                const Status*, hipStream_t);                                  \
   template void launch_cell_ranges<D>(int64_t, int64_t, const int*, int*, int*, hipStream_t);\
