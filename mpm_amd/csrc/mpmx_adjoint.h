@@ -69,12 +69,14 @@ struct AdjParticles {
 // adjoint runs in a separate pass over this compacted list: shear returns
 // from the front (count[0] entries), tensile ones from the back (count[1]
 // entries, slot cap - 1 down); per entry the particle id, the apex flag and
-// (SoA, stride cap) the strain increment, replaced by its adjoint.
+// (SoA, stride cap) the strain increment and the adjoints of the stress and
+// the strain increment (of those components that the dimension has).
 struct AdjList {
   int* count;
   int* ids;
   int* apex;
   double* buf;  // [6][cap]
+  double* out;  // [12][cap]
   int64_t cap;
 };
 

@@ -152,68 +152,50 @@ template <> struct Seeds<3> {
 };
 
 // Mohr-Coulomb: ls_in = J_s^T ls_out, lde = J_de^T ls_out, gE += dsigma/dE .
-// ls_out, gphi += dsigma/dphi . ls_out, by forward-mode passes of KC tangents.
+// ls_out, gphi += dsigma/dphi . ls_out: the pass of KC tangents from seed
+// `base` (Seeds' stress components, strain components, E, phi), acc[j] the
+// product of ls_out with the derivative for seed base + j.
 template <int D, int KC>
 MPMX_DEV void mc_vjp(const Material& m, double phi, double psi, double coh, double tcut,
-                     const double* s_in, const double* de, const double* ls_out, double* ls_in,
-                     double* lde, double& gE, double& gphi, bool frozen_flow) {
+                     const double* s_in, const double* de, const double* ls_out, int base,
+                     bool frozen_flow, double* acc) {
   using DT = ad::Dual<KC>;
   using Sd = Seeds<D>;
-  constexpr int NQ = Sd::NS + Sd::NE + 2;
-#pragma unroll 1
-  for (int base = 0; base < NQ; base += KC) {
-    DT S[6], E6[6];
+  DT S[6], E6[6];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      S[k] = ad::cst<DT>(s_in[k]);
-      E6[k] = ad::cst<DT>(de[k]);
+  for (int k = 0; k < 6; ++k) {
+    S[k] = ad::cst<DT>(s_in[k]);
+    E6[k] = ad::cst<DT>(de[k]);
+  }
+  ad::McParams<DT> P{ad::cst<DT>(m.a1), ad::cst<DT>(m.a2), ad::cst<DT>(m.G), ad::cst<DT>(phi),
+                     psi, coh, ad::cst<DT>(tcut), m.c_peak};
+#pragma unroll
+  for (int j = 0; j < KC; ++j) {
+    const int q = base + j;
+    if (q < Sd::NS) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+        if (k == Sd::s(q)) S[k].d[j] = 1.;
+    } else if (q < Sd::NS + Sd::NE) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+        if (k == Sd::e(q - Sd::NS)) E6[k].d[j] = 1.;
+    } else if (q == Sd::NS + Sd::NE) {
+      P.a1.d[j] = m.a1 / m.E;
+      P.a2.d[j] = m.a2 / m.E;
+      P.G.d[j] = m.G / m.E;
+    } else if (q == Sd::NS + Sd::NE + 1) {
+      P.phi.d[j] = 1.;
+      P.tcut.d[j] = m.dtcut_dphi;
     }
-    ad::McParams<DT> P{ad::cst<DT>(m.a1), ad::cst<DT>(m.a2), ad::cst<DT>(m.G), ad::cst<DT>(phi),
-                       psi, coh, ad::cst<DT>(tcut), m.c_peak};
+  }
+  DT O[6];
+  ad::mc_update(P, S, E6, O, frozen_flow);
 #pragma unroll
-    for (int j = 0; j < KC; ++j) {
-      const int q = base + j;
-      if (q >= NQ) break;
-      if (q < Sd::NS) {
+  for (int j = 0; j < KC; ++j) {
+    acc[j] = 0.;
 #pragma unroll
-        for (int k = 0; k < 6; ++k)
-          if (k == Sd::s(q)) S[k].d[j] = 1.;
-      } else if (q < Sd::NS + Sd::NE) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-          if (k == Sd::e(q - Sd::NS)) E6[k].d[j] = 1.;
-      } else if (q == Sd::NS + Sd::NE) {
-        P.a1.d[j] = m.a1 / m.E;
-        P.a2.d[j] = m.a2 / m.E;
-        P.G.d[j] = m.G / m.E;
-      } else {
-        P.phi.d[j] = 1.;
-        P.tcut.d[j] = m.dtcut_dphi;
-      }
-    }
-    DT O[6];
-    ad::mc_update(P, S, E6, O, frozen_flow);
-#pragma unroll
-    for (int j = 0; j < KC; ++j) {
-      const int q = base + j;
-      if (q >= NQ) break;
-      double acc = 0.;
-#pragma unroll
-      for (int i = 0; i < 6; ++i) acc += ls_out[i] * O[i].d[j];
-      if (q < Sd::NS) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-          if (k == Sd::s(q)) ls_in[k] = acc;
-      } else if (q < Sd::NS + Sd::NE) {
-#pragma unroll
-        for (int k = 0; k < 6; ++k)
-          if (k == Sd::e(q - Sd::NS)) lde[k] = acc;
-      } else if (q == Sd::NS + Sd::NE) {
-        gE += acc;
-      } else {
-        gphi += acc;
-      }
-    }
+    for (int i = 0; i < 6; ++i) acc[j] += ls_out[i] * O[i].d[j];
   }
 }
 
@@ -916,46 +898,62 @@ __global__ __launch_bounds__(kAdBlock) void k_ad_b5(Mesh M, Particles P, Slot s0
 }
 
 // The deferred plastic Mohr-Coulomb updates: constitutive adjoint by
-// forward-mode passes (stress adjoint and parameter gradients written; the
-// strain-increment adjoint left in Q.buf).
+// forward-mode passes of MPMX_AD_TANGENTS tangents (parameter gradients added;
+// the adjoints of the stress and the strain increment left in Q.out for
+// k_ad_mc_tail).
+// One thread per entry and pass, the passes' workgroups one after another: a
+// pass is a long dependent chain (the update's value is recomputed in each),
+// and a step of a few 10^4 plastic particles has too few entries to fill the
+// device with one thread each. 40 recorded steps and their backward pass, all
+// passes in one thread -> a thread each: 4.8k particles 13.5 -> 8.5 ms, 111k
+// 19.2 -> 13.0 ms, 1.05M 53.4 -> 48.7 ms (1 tangent a pass: 7.8, 13.4, 57.4).
 // One wave per workgroup: the waves' run times vary with their particles'
 // iteration counts, and a finished wave frees its slot at once.
 constexpr int kAdMcBlock = 64;
 template <int D>
+constexpr int kAdPasses = (Seeds<D>::NS + Seeds<D>::NE + 2 + MPMX_AD_TANGENTS - 1) /
+                          MPMX_AD_TANGENTS;
+template <int D>
 __global__ __launch_bounds__(kAdMcBlock) MPMX_AD_ATTR void k_ad_mc(Particles P,
                                                                    const Material* mats, Slot s0,
                                                                    AdjParticles L, AdjList Q) {
-  const int64_t e = blockIdx.x * (int64_t)kAdMcBlock + threadIdx.x;
+  using Sd = Seeds<D>;
+  constexpr int KC = MPMX_AD_TANGENTS;
   const int ns = Q.count[0];
-  if (e >= ns + Q.count[1]) return;
+  const int n = ns + Q.count[1];
+  const int nb = (n + kAdMcBlock - 1) / kAdMcBlock;
+  const int pass = nb > 0 ? (int)(blockIdx.x / nb) : kAdPasses<D>;
+  if (pass >= kAdPasses<D>) return;
+  const int64_t e = (int64_t)(blockIdx.x - pass * nb) * kAdMcBlock + threadIdx.x;
+  if (e >= n) return;
   const int64_t slot = e < ns ? e : Q.cap - 1 - (e - ns);
   const int64_t np = P.np;
   const int p = Q.ids[slot];
   const Material m = mats[stream_ld(&P.mat[p])];
-  double s_in[6], de[6], ls_out[6], ls_in[6], lde[6];
+  double s_in[6], de[6], ls_out[6], acc[KC];
 #pragma unroll
   for (int k = 0; k < 6; ++k) {
     s_in[k] = stream_ld(&s0.stress[k * np + p]);
     de[k] = Q.buf[k * Q.cap + slot];
     ls_out[k] = stream_ld(&L.ls[k * np + p]);
-    ls_in[k] = lde[k] = 0.;
   }
   const double phi = stream_ld(&P.sv[SV_PHI * np + p]), psi = stream_ld(&P.sv[SV_PSI * np + p]);
   const double coh = stream_ld(&P.sv[SV_COH * np + p]), tcut = stream_ld(&P.sv[SV_TCUT * np + p]);
-  double gE = 0., gphi = 0.;
-  mc_vjp<D, MPMX_AD_TANGENTS>(m, phi, psi, coh, tcut, s_in, de, ls_out, ls_in, lde, gE, gphi,
-                              Q.apex[slot] != 0);
+  mc_vjp<D, KC>(m, phi, psi, coh, tcut, s_in, de, ls_out, pass * KC, Q.apex[slot] != 0, acc);
 #pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    stream_st(&L.ls[k * np + p], ls_in[k]);
-    Q.buf[k * Q.cap + slot] = lde[k];
+  for (int j = 0; j < KC; ++j) {
+    const int q = pass * KC + j;
+    if (q < Sd::NS + Sd::NE)
+      Q.out[q * Q.cap + slot] = acc[j];
+    else if (q == Sd::NS + Sd::NE)
+      L.gE[p] += acc[j];
+    else if (q == Sd::NS + Sd::NE + 1)
+      L.gphi[p] += acc[j];
   }
-  L.gE[p] += gE;
-  L.gphi[p] += gphi;
 }
 
-// Their strain-increment adjoints through the velocity gradient: scatter
-// into lnv, shape adjoint into lxq.
+// Their stress adjoints, and the strain-increment adjoints through the
+// velocity gradient: scatter into lnv, shape adjoint into lxq.
 template <int D>
 __global__ __launch_bounds__(kAdBlock) void k_ad_mc_tail(Mesh M, Particles P, Slot s0,
                                                          const double* nv, double* lnv,
@@ -968,12 +966,20 @@ __global__ __launch_bounds__(kAdBlock) void k_ad_mc_tail(Mesh M, Particles P, Sl
   const int64_t slot = e < ns ? e : Q.cap - 1 - (e - ns);
   const int64_t np = P.np;
   const int p = Q.ids[slot];
+  using Sd = Seeds<D>;
+  double lde[6], ls_in[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) lde[k] = ls_in[k] = 0.;
+#pragma unroll
+  for (int q = 0; q < Sd::NS; ++q) ls_in[Sd::s(q)] = Q.out[q * Q.cap + slot];
+#pragma unroll
+  for (int q = 0; q < Sd::NE; ++q) lde[Sd::e(q)] = Q.out[(Sd::NS + q) * Q.cap + slot];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) stream_st(&L.ls[k * np + p], ls_in[k]);
   Shape<D> S;
   if (!load_shape<D>(M, s0, np, p, S)) return;
-  double v[NN][D], G[NN][D], lde[6], lxi[D];
+  double v[NN][D], G[NN][D], lxi[D];
   load_kinematics<D>(M, S, nv, v, G);
-#pragma unroll
-  for (int k = 0; k < 6; ++k) lde[k] = Q.buf[k * Q.cap + slot];
 #pragma unroll
   for (int k = 0; k < D; ++k) lxi[k] = 0.;
   double acc[NN][D];
@@ -1036,7 +1042,8 @@ static void backward_scheme(const Mesh& M, const Particles& P, const Nodes& Nd,
   const dim3 gp = ad_grid(P.np), gn = ad_grid(M.nnodes), b(kAdBlock);
   // the plastic Mohr-Coulomb updates queued by the stress pass
   auto plastic = [&](const double* nv, double* lnv) {
-    hipLaunchKernelGGL((k_ad_mc<D>), dim3((unsigned)((P.np + kAdMcBlock - 1) / kAdMcBlock)),
+    hipLaunchKernelGGL((k_ad_mc<D>),
+                       dim3((unsigned)((P.np + kAdMcBlock - 1) / kAdMcBlock * kAdPasses<D>)),
                        dim3(kAdMcBlock), 0, st, P, mats, s0, L, Q);
     hipLaunchKernelGGL((k_ad_mc_tail<D>), gp, b, 0, st, M, P, s0, nv, lnv, L, Q, a);
   };
