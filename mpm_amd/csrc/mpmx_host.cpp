@@ -814,7 +814,8 @@ void alloc_step_buffers(mpmx_ctx* c) {
   if (c->any_gn) c->d_rotF.alloc((size_t)(c->dim * 3 + c->dim * c->dim) * std::max<int64_t>(np, 1));
   if (c->any_mc_rate) c->d_plastic_trial.alloc(6 * std::max<int64_t>(np, 1));
   if (c->affine()) {
-    c->d_Cmat.alloc((size_t)c->dim * c->dim * std::max<int64_t>(np, 1));
+    if (c->flags & MPMX_ORDERED)
+      c->d_Cmat.alloc((size_t)c->dim * c->dim * std::max<int64_t>(np, 1));
     c->d_beta.alloc(std::max<int64_t>(np, 1));
   }
   if (c->any_mc) {
@@ -1105,7 +1106,7 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
     P.plastic_rec = B.plastic_rec;
   }
   if (P.spin) P.spin = B.spin;
-  if (P.Cmat) {
+  if (P.Bmat) {
     P.Cmat = B.Cmat;
     P.beta = B.beta;
   }
@@ -1134,14 +1135,18 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
   auto plastic = [&] {
     if (c->any_mc && !own) L("mc_plastic", [&] { launch_plastic(P, mats, S, st); });
   };
-  // affine velocity updates (APIC, ASFLIP, TPIC): the transfer matrix before
-  // each particle-to-grid map, the mapping matrix before grid-to-particle
+  // affine velocity updates (APIC, ASFLIP, TPIC): ordered mode's transfer
+  // matrix before each gather; the mapping matrix before a G2P with stress
+  // (and ASFLIP's before any)
   const bool aff = c->affine();
   auto affine = [&] {
     if (aff) L("affine_matrix", [&] { launch_affine_matrix<D>(M, P, c->vu, S, st); });
   };
   auto mapping = [&] {
     if (aff) L("mapping_matrix", [&] { launch_mapping_matrix<D>(M, P, Nd, A, c->vu, S, st); });
+  };
+  auto asflip = [&] {  // before a G2P without stress, which forms the others' itself
+    if (c->vu == ASFLIP) mapping();
   };
   if (full_sort || ordered)
     L("sort_by_cell", [&] {
@@ -1159,7 +1164,7 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       L("stress", [&] { launch_stress<D>(own, false, M, P, Nd, mats, A, S, scan, st); });
       plastic();
       L("gather_forces", [&] { launch_gather<D>(GK_F_ACC, M, P, Nd, A, S, perm, cs, ce, st); });
-      mapping();
+      asflip();
       L("g2p_locate", [&] { launch_g2p<D>(own, false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
     } else if (c->scheme == USL) {
       L("gather_all", [&] { launch_gather<D>(GK_ALL_VEL_ACC, M, P, Nd, A, S, perm, cs, ce, st); });
@@ -1168,7 +1173,7 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       plastic();
     } else {
       L("gather_all", [&] { launch_gather<D>(GK_ALL_VEL_ACC, M, P, Nd, A, S, perm, cs, ce, st); });
-      mapping();
+      asflip();
       L("g2p", [&] { launch_g2p<D>(own, false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
       affine();
       L("gather_momentum", [&] { launch_gather<D>(GK_MOM_VEL, M, P, Nd, A, S, perm, cs, ce, st); });
@@ -1176,14 +1181,13 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       plastic();
     }
   } else {
-    affine();
     if (c->scheme == USF) {
       L("p2g_mass_momentum", [&] { launch_p2g<D>(P2G_MV, c->chunk, M, P, Nd, A, S, perm, st); });
       L("node_velocity", [&] { launch_node<D>(ND_INIT | ND_VEL, M, Nd, A, S, st); });
       L("stress_force_scatter", [&] { launch_stress_scatter<D>(c->chunk, M, P, Nd, mats, A, S, perm, st); });
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_acceleration", [&] { launch_node<D>(ND_ACC | ND_ZERO_ALL, M, Nd, A, S, st); });
-      mapping();
+      asflip();
       L("g2p_locate", [&] { launch_g2p<D>(own, false, loc, M, P, Nd, mats, A, c->vu, S, scan, st); });
     } else if (c->scheme == USL) {
       L("p2g_all", [&] { launch_p2g<D>(P2G_MV_F, c->chunk, M, P, Nd, A, S, perm, st); });
@@ -1197,9 +1201,8 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       if (P.ntr > 0) L("traction_scatter", [&] { launch_traction_scatter<D>(M, P, Nd, S, st); });
       L("node_update", [&] { launch_node<D>(ND_INIT | ND_VEL | ND_ACC | ND_ZERO_MOM, M, Nd, A, S, st); });
       if (aff) {  // G2P, then the affine momentum map with the new positions
-        mapping();
+        asflip();
         L("g2p", [&] { launch_g2p<D>(own, false, false, M, P, Nd, mats, A, c->vu, S, scan, st); });
-        affine();
         L("p2g_momentum", [&] { launch_p2g<D>(P2G_MOM, c->chunk, M, P, Nd, A, S, perm, st); });
       } else {
         L("g2p_momentum_scatter", [&] { launch_g2p_scatter<D>(c->chunk, M, P, Nd, A, c->vu, S, perm, st); });
@@ -1244,6 +1247,7 @@ StepArgs step_args(const mpmx_ctx* c, double dt, double damping) {
   A.blending = c->blending;
   for (int k = 0; k < 3; ++k) A.g[k] = c->g[k];
   A.ramp = c->ramp;
+  A.vu = c->vu;
   A.ad_nodes = nullptr;
   A.ad_slot = nullptr;
   A.ad_stride = 0;
@@ -1266,12 +1270,7 @@ constexpr int64_t kGraphAfter = 24;
 void launch_steps(mpmx_ctx* c, int nsteps, double dt, double damping,
                   double* ad_nodes = nullptr, int64_t ad_stride = 0, int ad_nslots = 0) {
   const StepBuffers B = ctx_buffers(c);
-  StepArgs A;
-  A.dt = dt;
-  A.damping = damping;
-  A.blending = c->blending;
-  for (int k = 0; k < 3; ++k) A.g[k] = c->g[k];
-  A.ramp = c->ramp;
+  StepArgs A = step_args(c, dt, damping);
   A.ad_nodes = ad_nodes;
   A.ad_slot = ad_nodes ? &c->d_status.p->ad_slot : nullptr;
   A.ad_stride = ad_stride;
@@ -1470,7 +1469,8 @@ size_t carve_step_buffers(const mpmx_ctx* c, uintptr_t base, StepBuffers* B) {
   B->plastic_trial = c->any_mc_rate ? (double*)take(6 * np * sizeof(double)) : nullptr;
   B->Cmat = B->beta = nullptr;
   if (c->affine()) {
-    B->Cmat = (double*)take((size_t)c->dim * c->dim * np * sizeof(double));
+    if (c->flags & MPMX_ORDERED)
+      B->Cmat = (double*)take((size_t)c->dim * c->dim * np * sizeof(double));
     B->beta = (double*)take(np * sizeof(double));
   }
   return off;

@@ -175,8 +175,8 @@ struct Particles {
   // Affine velocity updates (APIC, ASFLIP, TPIC): the mapping matrix B
   // (mapping_matrix_, [D*D][np], row-major per particle) kept between steps;
   // the matrix C of the next particle-to-grid transfer ([D*D][np], momentum
-  // m N_i (v + C (x_i - x_p))); ASFLIP's beta of the step ([np]). Null for
-  // FLIP and PIC.
+  // m N_i (v + C (x_i - x_p)), ordered mode's gathers only); ASFLIP's beta of
+  // the step ([np], USL only). Null for FLIP and PIC.
   double* Bmat;
   double* Cmat;
   double* beta;
@@ -207,6 +207,7 @@ struct StepArgs {
   double blending;
   double g[3];
   double ramp;  // gravity ramping time (<= 0: none)
+  int vu;       // velocity update
   // Adjoint recording: when set, the node update kernels also store the
   // step's nodal quantities at ad_nodes + (*ad_slot) * ad_stride (layout:
   // mass [nn], then momentum, force, updated velocity, acceleration, MUSL

@@ -24,8 +24,9 @@ template <int D>
 void launch_locate_step(bool fast, const Mesh& M, const Particles& P, Status* S, int* scan_list,
                         hipStream_t st);
 // Affine velocity updates (APIC, ASFLIP, TPIC): the mapping matrices (and
-// ASFLIP's beta) before G2P; the matrix of the next particle-to-grid
-// transfer before each P2G.
+// ASFLIP's beta) before the G2P with the stress update (launch_g2p without it
+// forms APIC's and TPIC's itself); ordered mode's matrix of the next particle-to-grid
+// transfer before each gather (the scatters form it themselves).
 template <int D>
 void launch_mapping_matrix(const Mesh& M, const Particles& P, const Nodes& Nd,
                            const StepArgs& A, int vu, const Status* S, hipStream_t st);

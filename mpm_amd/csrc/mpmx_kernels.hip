@@ -654,6 +654,55 @@ MPMX_DEV void affine_velocity(const double* v, const double* C, const double* xp
   }
 }
 
+// The matrix C of the next affine particle-to-grid transfer, momentum
+// m N_i (v + C (x_i - x_p)); formed while staging (a kernel of its own and a
+// matrix per particle through HBM took 15 us per transfer, 237k particles; the
+// staging takes 3 more). C = B D^-1 with the shape tensor
+// D = sum_i N_i (x_i - x_p)(x_i - x_p)^T for APIC and ASFLIP
+// (map_mass_momentum_to_nodes_affine, particle.tcc:661-696), C = B for TPIC
+// (_taylor, :699-724). N at the particle's local coordinates, x_p its
+// current position.
+template <int D>
+MPMX_DEV void affine_matrix(const Mesh& M, const Particles& P, int vu, int64_t p, int c,
+                            const double* xi, const double* xp, double* C) {
+  constexpr int NN = Elem<D>::NN;
+  const int64_t np = P.np;
+  double B[D][D];
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b) C[a * D + b] = B[a][b] = P.Bmat[(a * D + b) * np + p];
+  if (vu == TPIC) return;
+  double N[NN], X[NN][D];
+  shapefn<D>(xi, N);
+  load_cell_X<D>(M, c, X);
+  double Dm[D][D], Di[D][D];
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b) Dm[a][b] = 0.;
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    double r[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) r[k] = X[i][k] - xp[k];
+#pragma unroll
+    for (int a = 0; a < D; ++a)
+#pragma unroll
+      for (int b = 0; b < D; ++b) Dm[a][b] = Dm[a][b] + (N[i] * r[a]) * r[b];
+  }
+  mat_inverse<D>(Dm, Di);
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b) {
+      double t = B[a][0] * Di[0][b];
+#pragma unroll
+      for (int k = 1; k < D; ++k) t = t + B[a][k] * Di[k][b];
+      C[a * D + b] = t;
+    }
+}
+
 // Internal force of a particle on node i (particle.tcc:914-950) is
 // f_i = -V (sigma . dN_i/dx) with dN_i/dx = J^-1 grad_i(xi), i.e.
 // f_i = B grad_i(xi) with B = -V sigma J^-1 (a DxD matrix per particle).
@@ -925,10 +974,12 @@ __global__ __launch_bounds__(CH) void k_p2g(Mesh M, Particles P, Nodes Nd, StepA
       }
       st.m[tid] = P.mass[p];
       if constexpr ((WHAT & SC_AFF) != 0) {
+        double xp[D], C[D * D];
 #pragma unroll
-        for (int k = 0; k < D * D; ++k) st.C[k][tid] = P.Cmat[k * np + p];
+        for (int k = 0; k < D; ++k) st.xp[k][tid] = xp[k] = stream_ld(&P.x[k * np + p]);
+        affine_matrix<D>(M, P, A.vu, p, key, xi, xp, C);
 #pragma unroll
-        for (int k = 0; k < D; ++k) st.xp[k][tid] = stream_ld(&P.x[k * np + p]);
+        for (int k = 0; k < D * D; ++k) st.C[k][tid] = C[k];
       }
       if constexpr ((WHAT & SC_F) != 0) {
         double sg[6];
@@ -1258,9 +1309,114 @@ __global__ __launch_bounds__(kStressBlock) MPMX_PRED_ATTR void k_stress(Mesh M, 
   }
 }
 
+// The mapping matrix of an affine velocity update at the start of G2P (before
+// the position xp moves), |B_ij| < 1e-15 -> 0, from the cell's nodal
+// velocities nv: compute_affine_mapping_matrix (particle.tcc:1687-1708),
+// B = sum_i N_i v_i (x_i - x_p)^T for APIC and ASFLIP, and
+// compute_velocity_gradient (:1662-1684), B = sum_i v_i dN_i/dx^T, for TPIC.
+// Returns ASFLIP's beta (compute_asflip_beta, :1711-1730): 0 when a node of
+// the cell has a velocity constraint or the deformation gradient increment of
+// the current nodal velocities compresses (det < 1), else 1.
+template <int D, int VU>
+MPMX_DEV double mapping_matrix(const Mesh& M, const Particles& P, const Nodes& Nd, double dt,
+                               int64_t p, int c, const double* xi, const double* xp,
+                               const double (*nv)[D]) {
+  constexpr int NN = Elem<D>::NN;
+  const int64_t np = P.np;
+  double B[D][D];
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b) B[a][b] = 0.;
+  double dndx[NN][D];
+  if constexpr (VU == TPIC || VU == ASFLIP) {
+    double Ji[D][D];
+    particle_dndx<D>(M, c, xi, dndx, Ji);
+  }
+  if constexpr (VU == TPIC) {
+#pragma unroll
+    for (int i = 0; i < NN; ++i)
+#pragma unroll
+      for (int a = 0; a < D; ++a)
+#pragma unroll
+        for (int b = 0; b < D; ++b) B[a][b] = B[a][b] + nv[i][a] * dndx[i][b];
+  } else {
+    double N[NN], X[NN][D];
+    shapefn<D>(xi, N);
+    load_cell_X<D>(M, c, X);
+#pragma unroll
+    for (int i = 0; i < NN; ++i)
+#pragma unroll
+      for (int a = 0; a < D; ++a)
+#pragma unroll
+        for (int b = 0; b < D; ++b) B[a][b] = B[a][b] + (N[i] * nv[i][a]) * (X[i][b] - xp[b]);
+  }
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b) P.Bmat[(a * D + b) * np + p] = fabs(B[a][b]) < 1.E-15 ? 0. : B[a][b];
+  if constexpr (VU != ASFLIP) return 0.;
+#pragma unroll
+  for (int i = 0; i < NN; ++i) {
+    const int n = M.cell_nodes[(int64_t)c * NN + i];
+    const int ci = Nd.cons ? Nd.cons[n] : -1;
+    if (ci >= 0 && Nd.table[ci].vmask != 0) return 0.;
+  }
+  double R[3][3] = {{1., 0., 0.}, {0., 1., 0.}, {0., 0., 1.}};
+#pragma unroll
+  for (int i = 0; i < NN; ++i)
+#pragma unroll
+    for (int a = 0; a < D; ++a)
+#pragma unroll
+      for (int b = 0; b < D; ++b) R[a][b] = R[a][b] + (nv[i][a] * dndx[i][b]) * dt;
+#pragma unroll
+  for (int a = 0; a < D; ++a)
+#pragma unroll
+    for (int b = 0; b < D; ++b) {
+      if (a != b && fabs(R[a][b]) < 1.E-15) R[a][b] = 0.;
+      if (a == b && fabs(R[a][b] - 1.) < 1.E-15) R[a][b] = 1.;
+    }
+  const double det = R[0][0] * (R[1][1] * R[2][2] - R[2][1] * R[1][2]) -
+                     R[1][0] * (R[0][1] * R[2][2] - R[2][1] * R[0][2]) +
+                     R[2][0] * (R[0][1] * R[1][2] - R[1][1] * R[0][2]);
+  return det < 1.0 ? 0.0 : 1.0;
+}
+
+// The same in a kernel of its own, before the G2P kernels that also update the
+// stress (USL), and for ASFLIP.
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_mapping_matrix(Mesh M, Particles P, Nodes Nd,
+                                                           StepArgs A, int vu,
+                                                           const Status* S) {
+  if (run_stopped(S)) return;
+  const int64_t p = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (p >= P.np) return;
+  const int64_t np = P.np;
+  const int c = P.cell[p];
+  if (!valid_cell<D>(M, c)) return;
+  double xi[D], xp[D];
+#pragma unroll
+  for (int k = 0; k < D; ++k) {
+    xi[k] = P.xi[k * np + p];
+    xp[k] = stream_ld(&P.x[k * np + p]);
+  }
+  double nv[Elem<D>::NN][D];
+  gather_nodes<D>(M, Nd, c, nv, nullptr);
+  if (vu == TPIC)
+    mapping_matrix<D, TPIC>(M, P, Nd, A.dt, p, c, xi, xp, nv);
+  else if (vu == APIC)
+    mapping_matrix<D, APIC>(M, P, Nd, A.dt, p, c, xi, xp, nv);
+  else
+    P.beta[p] = mapping_matrix<D, ASFLIP>(M, P, Nd, A.dt, p, c, xi, xp, nv);
+}
+
 // G2P: compute_updated_position (particle.tcc:994-1070) in particle order,
-// optionally followed by the USL stress update and by locate.
-template <int D, bool STRESS, bool LOCATE, bool ROT = false>
+// optionally followed by the USL stress update and by locate. AFF: the affine
+// velocity update (APIC, TPIC) whose mapping matrix is formed here first
+// (FLIP: none). APIC, 237k particles in 3D: mapping 15.4 + G2P 17.2 us -> 22.4
+// in one; ASFLIP's beta on top would spill (58 registers), so it keeps a
+// mapping kernel of its own.
+template <int D, bool STRESS, bool LOCATE, bool ROT = false, int AFF = FLIP>
 __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_g2p(Mesh M, Particles P, Nodes Nd,
                                                 const Material* mats, StepArgs A, int vu,
                                                 Status* S, int* scan_list) {
@@ -1296,7 +1452,11 @@ __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_g2p(Mesh M, Particles
     u0[k] = stream_ld(&P.u[k * np + p]);
   }
   const int pvc = P.pvc_mask ? P.pvc_mask[p] : 0;
-  const double beta = vu == ASFLIP ? P.beta[p] : 0.;
+  double beta = 0.;
+  if constexpr (AFF != FLIP)
+    beta = mapping_matrix<D, AFF>(M, P, Nd, A.dt, p, c, xi, x, nv);
+  else if (vu == ASFLIP)
+    beta = P.beta[p];
 #pragma unroll
   for (int k = 0; k < D; ++k) {
     double v, dx;
@@ -1316,158 +1476,26 @@ __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_g2p(Mesh M, Particles
   if constexpr (LOCATE) locate_one<D>(M, P, S, scan_list, (int)p, x, c, -1);
 }
 
-// The mapping matrices of the affine velocity updates at the start of G2P
-// (before the positions move), |B_ij| < 1e-15 -> 0:
-// compute_affine_mapping_matrix (particle.tcc:1687-1708),
-// B = sum_i N_i v_i (x_i - x_p)^T for APIC and ASFLIP, and
-// compute_velocity_gradient (:1662-1684), B = sum_i v_i dN_i/dx^T, for TPIC.
-// ASFLIP also gets its beta (compute_asflip_beta, :1711-1730): 0 when a node
-// of the cell has a velocity constraint or the deformation gradient
-// increment of the current nodal velocities compresses (det < 1), else 1.
-template <int D>
-__global__ __launch_bounds__(kBlock) void k_mapping_matrix(Mesh M, Particles P, Nodes Nd,
-                                                           StepArgs A, int vu,
-                                                           const Status* S) {
-  if (run_stopped(S)) return;
-  constexpr int NN = Elem<D>::NN;
-  const int64_t p = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-  if (p >= P.np) return;
-  const int64_t np = P.np;
-  const int c = P.cell[p];
-  if (!valid_cell<D>(M, c)) return;
-  double xi[D], xp[D];
-#pragma unroll
-  for (int k = 0; k < D; ++k) {
-    xi[k] = P.xi[k * np + p];
-    xp[k] = stream_ld(&P.x[k * np + p]);
-  }
-  double nv[NN][D];
-  gather_nodes<D>(M, Nd, c, nv, nullptr);
-  double B[D][D];
-#pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int b = 0; b < D; ++b) B[a][b] = 0.;
-  double dndx[NN][D];
-  if (vu == TPIC || vu == ASFLIP) {
-    double Ji[D][D];
-    particle_dndx<D>(M, c, xi, dndx, Ji);
-  }
-  if (vu == TPIC) {
-#pragma unroll
-    for (int i = 0; i < NN; ++i)
-#pragma unroll
-      for (int a = 0; a < D; ++a)
-#pragma unroll
-        for (int b = 0; b < D; ++b) B[a][b] = B[a][b] + nv[i][a] * dndx[i][b];
-  } else {
-    double N[NN], X[NN][D];
-    shapefn<D>(xi, N);
-    load_cell_X<D>(M, c, X);
-#pragma unroll
-    for (int i = 0; i < NN; ++i)
-#pragma unroll
-      for (int a = 0; a < D; ++a)
-#pragma unroll
-        for (int b = 0; b < D; ++b) B[a][b] = B[a][b] + (N[i] * nv[i][a]) * (X[i][b] - xp[b]);
-  }
-#pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int b = 0; b < D; ++b) P.Bmat[(a * D + b) * np + p] = fabs(B[a][b]) < 1.E-15 ? 0. : B[a][b];
-  if (vu != ASFLIP) return;
-  double beta = 1.0;
-#pragma unroll
-  for (int i = 0; i < NN; ++i) {
-    const int n = M.cell_nodes[(int64_t)c * NN + i];
-    const int ci = Nd.cons ? Nd.cons[n] : -1;
-    if (ci >= 0 && Nd.table[ci].vmask != 0) beta = 0.0;
-  }
-  if (beta != 0.0) {
-    double R[3][3] = {{1., 0., 0.}, {0., 1., 0.}, {0., 0., 1.}};
-#pragma unroll
-    for (int i = 0; i < NN; ++i)
-#pragma unroll
-      for (int a = 0; a < D; ++a)
-#pragma unroll
-        for (int b = 0; b < D; ++b) R[a][b] = R[a][b] + (nv[i][a] * dndx[i][b]) * A.dt;
-#pragma unroll
-    for (int a = 0; a < D; ++a)
-#pragma unroll
-      for (int b = 0; b < D; ++b) {
-        if (a != b && fabs(R[a][b]) < 1.E-15) R[a][b] = 0.;
-        if (a == b && fabs(R[a][b] - 1.) < 1.E-15) R[a][b] = 1.;
-      }
-    const double det = R[0][0] * (R[1][1] * R[2][2] - R[2][1] * R[1][2]) -
-                       R[1][0] * (R[0][1] * R[2][2] - R[2][1] * R[0][2]) +
-                       R[2][0] * (R[0][1] * R[1][2] - R[1][1] * R[0][2]);
-    if (det < 1.0) beta = 0.0;
-  }
-  P.beta[p] = beta;
-}
-
-// The matrix C of the next affine particle-to-grid transfer, momentum
-// m N_i (v + C (x_i - x_p)): C = B D^-1 with the shape tensor
-// D = sum_i N_i (x_i - x_p)(x_i - x_p)^T for APIC and ASFLIP
-// (map_mass_momentum_to_nodes_affine, particle.tcc:661-696), C = B for TPIC
-// (_taylor, :699-724). N at the particle's local coordinates, x_p its
-// current position.
+// Ordered mode: the matrices of the next affine transfer, for the gathers (fast
+// mode's scatters form them while staging).
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_affine_matrix(Mesh M, Particles P, int vu,
                                                           const Status* S) {
   if (run_stopped(S)) return;
-  constexpr int NN = Elem<D>::NN;
   const int64_t p = blockIdx.x * (int64_t)kBlock + threadIdx.x;
   if (p >= P.np) return;
   const int64_t np = P.np;
   const int c = P.cell[p];
   if (!valid_cell<D>(M, c)) return;
-  double B[D][D];
-#pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int b = 0; b < D; ++b) B[a][b] = P.Bmat[(a * D + b) * np + p];
-  if (vu == TPIC) {
-#pragma unroll
-    for (int a = 0; a < D; ++a)
-#pragma unroll
-      for (int b = 0; b < D; ++b) P.Cmat[(a * D + b) * np + p] = B[a][b];
-    return;
-  }
-  double xi[D], xp[D];
+  double xi[D], xp[D], C[D * D];
 #pragma unroll
   for (int k = 0; k < D; ++k) {
     xi[k] = P.xi[k * np + p];
     xp[k] = stream_ld(&P.x[k * np + p]);
   }
-  double N[NN], X[NN][D];
-  shapefn<D>(xi, N);
-  load_cell_X<D>(M, c, X);
-  double Dm[D][D], Di[D][D];
+  affine_matrix<D>(M, P, vu, p, c, xi, xp, C);
 #pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int b = 0; b < D; ++b) Dm[a][b] = 0.;
-#pragma unroll
-  for (int i = 0; i < NN; ++i) {
-    double r[D];
-#pragma unroll
-    for (int k = 0; k < D; ++k) r[k] = X[i][k] - xp[k];
-#pragma unroll
-    for (int a = 0; a < D; ++a)
-#pragma unroll
-      for (int b = 0; b < D; ++b) Dm[a][b] = Dm[a][b] + (N[i] * r[a]) * r[b];
-  }
-  mat_inverse<D>(Dm, Di);
-#pragma unroll
-  for (int a = 0; a < D; ++a)
-#pragma unroll
-    for (int b = 0; b < D; ++b) {
-      double t = B[a][0] * Di[0][b];
-#pragma unroll
-      for (int k = 1; k < D; ++k) t = t + B[a][k] * Di[k][b];
-      P.Cmat[(a * D + b) * np + p] = t;
-    }
+  for (int k = 0; k < D * D; ++k) P.Cmat[k * np + p] = C[k];
 }
 
 // The deferred Mohr-Coulomb return mappings of this step: the rest of
@@ -2241,7 +2269,7 @@ template <int D>
 void launch_p2g(int what, int chunk, const Mesh& M, const Particles& P, const Nodes& Nd,
                 const StepArgs& A, const Status* S, const int* perm,
                 hipStream_t st) {
-  if (P.Cmat) {  // affine velocity updates: 128-particle chunks
+  if (P.Bmat) {  // affine velocity updates: 128-particle chunks
     if (what == SC_MV)
       MPMX_LAUNCH_CH(128, (k_p2g<D, SC_MV | SC_AFF, 128>), P.np, st, M, P, Nd, A, S, perm);
     else if (what == SC_MOM)
@@ -2363,6 +2391,16 @@ void launch_g2p(bool fast, bool stress, bool locate, const Mesh& M, const Partic
     MPMX_LAUNCH((k_g2p<D, true, false, true>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
   else if (stress)
     MPMX_LAUNCH((k_g2p<D, true, false>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
+#define MPMX_G2P_AFFINE(VU)                                                                       \
+  else if (vu == VU && locate)                                                                   \
+    MPMX_LAUNCH((k_g2p<D, false, true, false, VU>), P.np, st, M, P, Nd, mats, A, vu, S,          \
+                scan_list);                                                                      \
+  else if (vu == VU)                                                                             \
+    MPMX_LAUNCH((k_g2p<D, false, false, false, VU>), P.np, st, M, P, Nd, mats, A, vu, S,         \
+                scan_list);
+  MPMX_G2P_AFFINE(APIC)
+  MPMX_G2P_AFFINE(TPIC)
+#undef MPMX_G2P_AFFINE
   else if (locate)
     MPMX_LAUNCH((k_g2p<D, false, true>), P.np, st, M, P, Nd, mats, A, vu, S, scan_list);
   else
