@@ -225,6 +225,12 @@ struct mpmx_ctx {
   void* scratch = nullptr;
   std::string scratch_error;
 
+  // staging of the particle read-back (read_rows)
+  DBuf<char> d_read;
+  char* h_read = nullptr;  // pinned
+  size_t read_bytes = 0;   // of each of the two halves
+  hipEvent_t read_done[2] = {nullptr, nullptr};
+
   // profiling
   bool profile = false;
   std::vector<std::string> kt_names;
@@ -234,6 +240,9 @@ struct mpmx_ctx {
     for (auto& g : graph_exec)
       if (g) (void)hipGraphExecDestroy(g);
     if (h_status) (void)hipHostFree(h_status);
+    if (h_read) (void)hipHostFree(h_read);
+    for (auto e : read_done)
+      if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -735,6 +744,84 @@ void get_soa(const DBuf<T>& b, int64_t np, int comps, T* rows, hipStream_t st) {
     HIPCHECK(hipStreamSynchronize(st));
     for (int64_t i = 0; i < np; ++i) rows[i * comps + k] = col[i];
   }
+}
+
+// One array to read back: component-major on the device, rows on the host.
+struct ReadField {
+  const void* in;
+  char* out;
+  int comps, kind, size;
+};
+
+// Copies fields of n particles to the host: packed into rows by a kernel, a
+// piece of the staging at a time, each piece one copy to pinned memory while
+// the piece before it is spread to the caller's arrays. (A copy per component
+// and a transposition on the host took 0.5 ms for 8192 particles, most of it
+// the 63 copies' latency.) The staging, twice the size of the largest read so
+// far and at most 2 x 4 MiB on each side, stays the context's.
+void read_rows(mpmx_ctx* c, const std::vector<ReadField>& f, int64_t n) {
+  if (f.empty()) return;
+  size_t want = size_t(64) << 10, total = 0;
+  for (const auto& q : f) total += (size_t)q.comps * q.size * n + 16;
+  while (want < total && want < (size_t(4) << 20)) want *= 2;
+  if (c->read_bytes < want) {
+    if (c->h_read) (void)hipHostFree(c->h_read);
+    c->h_read = nullptr;
+    c->read_bytes = 0;
+    c->d_read.alloc(2 * want);
+    HIPCHECK(hipHostMalloc((void**)&c->h_read, 2 * want));
+    c->read_bytes = want;
+    for (auto& e : c->read_done)
+      if (!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  const size_t side_bytes = c->read_bytes;
+  struct Piece {
+    const ReadField* f;
+    int64_t r0, rows;
+    size_t off;
+  };
+  std::vector<Piece> pieces[2];
+  auto spread = [&](int side) {
+    if (pieces[side].empty()) return;
+    HIPCHECK(hipEventSynchronize(c->read_done[side]));
+    for (const Piece& p : pieces[side]) {
+      const size_t row = (size_t)p.f->comps * p.f->size;
+      std::memcpy(p.f->out + p.r0 * row, c->h_read + side * side_bytes + p.off, p.rows * row);
+    }
+    pieces[side].clear();
+  };
+  size_t k = 0;
+  int64_t r0 = 0;
+  for (int side = 0; k < f.size(); side ^= 1) {
+    spread(side);
+    PackTable T;
+    T.count = 0;
+    size_t used = 0;
+    while (k < f.size() && T.count < PackTable::kMax) {
+      const size_t row = (size_t)f[k].comps * f[k].size;
+      const int64_t rows = std::min<int64_t>(n - r0, (int64_t)((side_bytes - used) / row));
+      if (rows <= 0) break;
+      T.e[T.count++] = {f[k].in, c->d_read.p + side * side_bytes + used, r0, rows, f[k].comps,
+                        f[k].kind};
+      pieces[side].push_back({&f[k], r0, rows, used});
+      used = (used + rows * row + 15) & ~size_t(15);
+      r0 += rows;
+      if (r0 < n || used >= side_bytes) break;
+      r0 = 0;
+      ++k;
+    }
+    if (r0 == n) {
+      r0 = 0;
+      ++k;
+    }
+    launch_pack_rows(T, n, c->stream);
+    HIPCHECK(hipGetLastError());
+    HIPCHECK(hipMemcpyAsync(c->h_read + side * side_bytes, c->d_read.p + side * side_bytes, used,
+                            hipMemcpyDeviceToHost, c->stream));
+    HIPCHECK(hipEventRecord(c->read_done[side], c->stream));
+  }
+  spread(0);
+  spread(1);
 }
 
 // Per-particle mask and values of the particle velocity constraints, in the
@@ -2281,31 +2368,29 @@ int mpmx_get_particles(mpmx_ctx* c, double* x, double* u, double* v, double* str
   API_BEGIN(c)
   const int64_t np = c->np;
   const int d = c->dim;
-  hipStream_t st = c->stream;
-  HIPCHECK(hipStreamSynchronize(st));
+  HIPCHECK(hipStreamSynchronize(c->stream));
   if (np == 0) return MPMX_OK;
-  if (x) get_soa(c->d_x, np, d, x, st);
-  if (u) get_soa(c->d_u, np, d, u, st);
-  if (v) get_soa(c->d_v, np, d, v, st);
-  if (stress) get_soa(c->d_stress, np, 6, stress, st);
-  if (strain) get_soa(c->d_strain, np, 6, strain, st);
-  if (F) get_soa(c->d_F, np, 9, F, st);
-  if (mass) get_soa(c->d_mass, np, 1, mass, st);
-  if (volume) get_soa(c->d_vol, np, 1, volume, st);
-  if (density) get_soa(c->d_rho, np, 1, density, st);
-  if (material_id) get_soa(c->d_mat, np, 1, material_id, st);
-  if (xi) get_soa(c->d_xi, np, d, xi, st);
-  if (cell) {
-    std::vector<int> cc(np);
-    get_soa(c->d_cell, np, 1, cc.data(), st);
-    for (int64_t i = 0; i < np; ++i) cell[i] = cc[i];
-  }
-  if (statevars) {
-    if (c->any_mc)
-      get_soa(c->d_sv, np, NSV, statevars, st);
-    else
-      std::fill(statevars, statevars + np * NSV, 0.0);
-  }
+  std::vector<ReadField> f;
+  auto add = [&](const void* in, void* out, int comps, int kind = PACK_F64) {
+    if (out) f.push_back({in, (char*)out, comps, kind, kind == PACK_I32 ? 4 : 8});
+  };
+  add(c->d_x.p, x, d);
+  add(c->d_u.p, u, d);
+  add(c->d_v.p, v, d);
+  add(c->d_stress.p, stress, 6);
+  add(c->d_strain.p, strain, 6);
+  add(c->d_F.p, F, 9);
+  add(c->d_mass.p, mass, 1);
+  add(c->d_vol.p, volume, 1);
+  add(c->d_rho.p, density, 1);
+  add(c->d_mat.p, material_id, 1, PACK_I32);
+  add(c->d_xi.p, xi, d);
+  add(c->d_cell.p, cell, 1, PACK_I64);
+  if (statevars && c->any_mc)
+    add(c->d_sv.p, statevars, NSV);
+  else if (statevars)
+    std::fill(statevars, statevars + np * NSV, 0.0);
+  read_rows(c, f, np);
   API_END(c)
 }
 

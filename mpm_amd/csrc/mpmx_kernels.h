@@ -93,6 +93,22 @@ void launch_gather(int which, const Mesh& M, const Particles& P, const Nodes& Nd
 template <int D>
 void launch_rows_xv(const Particles& P, double* rx, double* rv, hipStream_t st);
 
+// Copies of rows of component-major arrays (double, int, or int widened to
+// 64 bits) into row-major ones.
+enum { PACK_F64 = 0, PACK_I32 = 1, PACK_I64 = 2 };
+struct PackEntry {
+  const void* in;  // [comps][n]
+  void* out;       // [rows][comps]
+  int64_t r0, rows;
+  int comps, kind;
+};
+struct PackTable {
+  static constexpr int kMax = 16;
+  int count;
+  PackEntry e[kMax];
+};
+void launch_pack_rows(const PackTable& T, int64_t n, hipStream_t st);
+
 // out[k * nnew + i] = in[k * nold + idx[i]] for the comps components of a
 // component-major array (T = double or int).
 template <class T>

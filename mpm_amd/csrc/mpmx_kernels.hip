@@ -2485,6 +2485,31 @@ void launch_rows_xv(const Particles& P, double* rx, double* rv, hipStream_t st) 
   MPMX_LAUNCH((k_rows_xv<D>), P.np, st, P.x, P.v, rx, rv, P.np);
 }
 
+// Rows of component-major arrays, for reading state back: each table entry
+// copies `rows` rows from row r0 of an array of n to `out` (row-major).
+__global__ __launch_bounds__(kBlock) void k_pack_rows(PackTable T, int64_t n) {
+  const PackEntry& f = T.e[blockIdx.y];
+  const int64_t total = f.rows * f.comps;
+  for (int64_t j = blockIdx.x * (int64_t)kBlock + threadIdx.x; j < total;
+       j += (int64_t)gridDim.x * kBlock) {
+    const int64_t i = j / f.comps, k = j - i * f.comps, src = k * n + f.r0 + i;
+    if (f.kind == PACK_F64)
+      ((double*)f.out)[j] = ((const double*)f.in)[src];
+    else if (f.kind == PACK_I32)
+      ((int*)f.out)[j] = ((const int*)f.in)[src];
+    else
+      ((int64_t*)f.out)[j] = ((const int*)f.in)[src];
+  }
+}
+void launch_pack_rows(const PackTable& T, int64_t n, hipStream_t st) {
+  if (T.count <= 0) return;
+  int64_t most = 1;
+  for (int i = 0; i < T.count; ++i) most = std::max(most, T.e[i].rows * T.e[i].comps);
+  const int64_t blocks = std::min<int64_t>((most + kBlock - 1) / kBlock, 1024);
+  hipLaunchKernelGGL(k_pack_rows, dim3((unsigned)blocks, (unsigned)T.count), dim3(kBlock), 0, st,
+                     T, n);
+}
+
 template <class T>
 void take_rows(const T* in, T* out, const int* idx, int64_t nnew, int64_t nold, int comps,
                hipStream_t st) {
