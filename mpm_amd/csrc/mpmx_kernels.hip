@@ -1784,9 +1784,9 @@ __global__ __launch_bounds__(kBlock) void k_cell_ranges(int64_t np, int64_t ncel
   if (k == np - 1 || skey[k + 1] != c) cend[c] = (int)k + 1;
 }
 
-__global__ void k_fill_int(int* a, int64_t n, int v) {
+__global__ void k_clear_pair(int* a, int* b, int64_t n) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i < n) a[i] = v;
+  if (i < n) a[i] = b[i] = 0;
 }
 
 // Per node: the particles of its cells summed in particle-id order (the
@@ -2435,10 +2435,8 @@ void launch_node(int fl, const Mesh& M, const Nodes& Nd, const StepArgs& A, cons
 template <int D>
 void launch_cell_ranges(int64_t np, int64_t ncells, const int* skey, int* cstart, int* cend,
                         hipStream_t st) {
-  if (ncells > 0) {
-    hipLaunchKernelGGL(k_fill_int, grid_for(ncells), dim3(kBlock), 0, st, cstart, ncells, 0);
-    hipLaunchKernelGGL(k_fill_int, grid_for(ncells), dim3(kBlock), 0, st, cend, ncells, 0);
-  }
+  if (ncells > 0)
+    hipLaunchKernelGGL(k_clear_pair, grid_for(ncells), dim3(kBlock), 0, st, cstart, cend, ncells);
   MPMX_LAUNCH((k_cell_ranges<D>), np, st, np, ncells, skey, cstart, cend);
 }
 

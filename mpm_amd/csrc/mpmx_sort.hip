@@ -1,61 +1,81 @@
-// Stable LSD radix sort of particles by cell id (8-bit digits).
+// Stable LSD radix sort of particles by cell id.
 //
 // Binning (locate_particles, mesh.tcc:1097-1153) gives each particle a cell;
 // the scatter kernels need the particles grouped by cell with ascending
 // particle ids inside each cell. Sorting the pairs (cell, id) with a stable
 // sort over the id-ordered input gives exactly that. Each pass is
-//   hist:    per 4096-key tile, a 256-bin digit histogram (LDS atomics),
+//   hist:    per tile, a digit histogram (LDS atomics),
 //   scan:    exclusive scan of the digit-major histogram table,
-//   scatter: per tile, stable ranks from wave64 ballots (8 one-bit ballots
+//   scatter: per tile, stable ranks from wave64 ballots (one-bit ballots
 //            form each lane's digit-match mask), written at the scanned
 //            offsets.
+// The first pass reads the particles' cells themselves. A pass costs launches
+// and tile latency rather than bytes at the sizes a step has, so digits are as
+// wide as makes the passes few (up to 10 bits: 2 passes up to a million cells,
+// where 8-bit digits took 3), and tiles shrink with the number of particles so
+// that they still cover the device. One sort with 8-bit digits, 4096-key tiles
+// and 5 launches a pass -> this: 8k particles 67 -> 26 us, 24k 64 -> 34, 262k
+// (3 passes -> 2) 96 -> 42, 2.1M 133 -> 103, 5.2M 180 -> 140.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "mpmx_kernels.h"
 
 namespace mpmx {
 
 static constexpr int kSortBlock = 256;
-static constexpr int kRounds = 16;
-static constexpr int kTile = kSortBlock * kRounds;
 static constexpr int kWaves = kSortBlock / 64;
+static constexpr int kMaxBits = 10;
+static constexpr int kMaxBins = 1 << kMaxBits;
 static constexpr int kScanTile = 1024;
+// Up to this many table entries one workgroup scans the table in one launch.
+static constexpr int kScanOne = 32768;
+// Up to this many scan tiles, every tile sums the totals before it itself.
+static constexpr int kScanDirect = 2048;
 
-static inline int64_t tiles_for(int64_t n) { return (n + kTile - 1) / kTile; }
+// Rounds of kSortBlock keys per tile: short tiles for few particles (a tile is
+// a chain of dependent rounds, 1 us each), long ones where the table, a row of
+// digits per tile, would cost more than the rounds.
+static inline int rounds_for(int64_t n) {
+  return n < (64 << 10) ? 1 : (n < (512 << 10) ? 4 : (n < (2 << 20) ? 8 : 16));
+}
+static inline int64_t tiles_for(int64_t n) {
+  const int64_t t = (int64_t)kSortBlock * rounds_for(n);
+  return (n + t - 1) / t;
+}
 
 int64_t radix_sort_temp_ints(int64_t n) {
-  const int64_t nb = tiles_for(n) > 0 ? tiles_for(n) : 1;
-  const int64_t nt = (256 * nb + kScanTile - 1) / kScanTile;
-  return 4 * n + 256 * nb + nt + 64;
+  const int64_t nb = std::max<int64_t>(tiles_for(n), 1);
+  return 2 * n + kMaxBins * nb + (kMaxBins * nb + kScanTile - 1) / kScanTile + 64;
 }
 
-// keys: cell in [0, ncells) else max_key; values: particle id
-__global__ __launch_bounds__(kSortBlock) void k_rs_init(const int* cell, int64_t n, int max_key,
-                                                        int* keys, int* vals) {
-  const int64_t i = blockIdx.x * (int64_t)kSortBlock + threadIdx.x;
-  if (i >= n) return;
-  const int c = cell[i];
-  keys[i] = (c >= 0 && c < max_key) ? c : max_key;
-  vals[i] = (int)i;
+// keys: cell in [0, ncells) else max_key
+template <bool FIRST>
+__device__ __forceinline__ int load_key(const int* keys, int64_t i, int max_key) {
+  const int c = keys[i];
+  return !FIRST || (c >= 0 && c < max_key) ? c : max_key;
 }
 
-__global__ __launch_bounds__(kSortBlock) void k_rs_hist(const int* keys, int64_t n, int shift,
+template <bool FIRST>
+__global__ __launch_bounds__(kSortBlock) void k_rs_hist(const int* keys, int64_t n, int max_key,
+                                                        int shift, int nbins, int rounds,
                                                         int* hist, int64_t nblocks) {
-  __shared__ int bins[256];
-  bins[threadIdx.x] = 0;
+  __shared__ int bins[kMaxBins];
+  for (int b = threadIdx.x; b < nbins; b += kSortBlock) bins[b] = 0;
   __syncthreads();
-  const int64_t base = blockIdx.x * (int64_t)kTile;
-  for (int r = 0; r < kRounds; ++r) {
+  const int64_t base = blockIdx.x * (int64_t)(kSortBlock * rounds);
+  for (int r = 0; r < rounds; ++r) {
     const int64_t i = base + r * kSortBlock + threadIdx.x;
-    if (i < n) atomicAdd(&bins[(keys[i] >> shift) & 255], 1);
+    if (i < n) atomicAdd(&bins[(load_key<FIRST>(keys, i, max_key) >> shift) & (nbins - 1)], 1);
   }
   __syncthreads();
-  hist[threadIdx.x * nblocks + blockIdx.x] = bins[threadIdx.x];
+  for (int b = threadIdx.x; b < nbins; b += kSortBlock) hist[b * nblocks + blockIdx.x] = bins[b];
 }
 
 // Exclusive scan of `total` ints in place: each 1024-element tile is scanned
 // by one block (4 consecutive elements per thread, wave prefix sums by
-// shuffles), tile totals are scanned by one block, then added back.
+// shuffles), then the totals of the tiles before it are added.
 
 __device__ __forceinline__ int wave_incl_scan(int v) {
   const int lane = threadIdx.x & 63;
@@ -67,23 +87,43 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   return v;
 }
 
-// block-wide exclusive scan of one value per thread (256 threads); returns
-// the exclusive prefix and writes the block total to *total
+// block-wide exclusive scan of one value per thread (WAVES * 64 threads);
+// returns the exclusive prefix and writes the block total to *total
+template <int WAVES>
 __device__ __forceinline__ int block_excl_scan(int v, int* total) {
-  __shared__ int wsum[4];
+  __shared__ int wsum[WAVES];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int incl = wave_incl_scan(v);
   if (lane == 63) wsum[wave] = incl;
   __syncthreads();
   int before = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < WAVES; ++w) {
     before += (w < wave) ? wsum[w] : 0;
     tot += wsum[w];
   }
   __syncthreads();
   *total = tot;
   return before + incl - v;
+}
+
+// The whole table (at most kScanOne entries) by one workgroup.
+__global__ __launch_bounds__(1024) void k_rs_scan_one(int* a, int total) {
+  constexpr int PER = kScanOne / 1024;
+  const int per = (total + 1023) / 1024, b = threadIdx.x * per;
+  int v[PER], s = 0;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    v[j] = (j < per && b + j < total) ? a[b + j] : 0;
+    s += v[j];
+  }
+  int tot;
+  int run = block_excl_scan<16>(s, &tot);
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if (j < per && b + j < total) a[b + j] = run;
+    run += v[j];
+  }
 }
 
 __global__ __launch_bounds__(256) void k_rs_scan_tiles(int* a, int64_t total, int* tile_sums) {
@@ -93,7 +133,7 @@ __global__ __launch_bounds__(256) void k_rs_scan_tiles(int* a, int64_t total, in
   for (int j = 0; j < 4; ++j) v[j] = (base + j < total) ? a[base + j] : 0;
   const int s = (v[0] + v[1]) + (v[2] + v[3]);
   int tot;
-  int run = block_excl_scan(s, &tot);
+  int run = block_excl_scan<4>(s, &tot);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (base + j < total) a[base + j] = run;
@@ -111,7 +151,7 @@ __global__ __launch_bounds__(256) void k_rs_scan_sums(int* sums, int64_t n) {
     const int64_t i = b + threadIdx.x;
     const int v = i < n ? sums[i] : 0;
     int tot;
-    const int ex = block_excl_scan(v, &tot);
+    const int ex = block_excl_scan<4>(v, &tot);
     if (i < n) sums[i] = carry + ex;
     __syncthreads();
     if (threadIdx.x == 0) carry += tot;
@@ -119,8 +159,18 @@ __global__ __launch_bounds__(256) void k_rs_scan_sums(int* sums, int64_t n) {
   }
 }
 
+// DIRECT: `sums` holds the tiles' totals, summed here up to the block's own;
+// else their exclusive scan.
+template <bool DIRECT>
 __global__ __launch_bounds__(256) void k_rs_scan_add(int* a, int64_t total, const int* sums) {
-  const int add = sums[blockIdx.x];
+  int add = 0;
+  if constexpr (DIRECT) {
+    int s = 0;
+    for (int i = threadIdx.x; i < (int)blockIdx.x; i += 256) s += sums[i];
+    (void)block_excl_scan<4>(s, &add);
+  } else {
+    add = sums[blockIdx.x];
+  }
   const int64_t base = blockIdx.x * (int64_t)kScanTile;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -129,38 +179,42 @@ __global__ __launch_bounds__(256) void k_rs_scan_add(int* a, int64_t total, cons
   }
 }
 
+template <bool FIRST>
 __global__ __launch_bounds__(kSortBlock) void k_rs_scatter(const int* kin, const int* vin,
                                                            int* kout, int* vout, int64_t n,
-                                                           int shift, const int* hist,
+                                                           int max_key, int shift, int bits,
+                                                           int rounds, const int* hist,
                                                            int64_t nblocks) {
-  __shared__ int base[256];
-  __shared__ int wcount[kWaves][256];
+  __shared__ int base[kMaxBins];
+  __shared__ unsigned short wcount[kWaves][kMaxBins];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  base[tid] = hist[tid * nblocks + blockIdx.x];
-  const unsigned long long lt = (1ull << lane) - 1ull;
-  const int64_t tbase = blockIdx.x * (int64_t)kTile;
-  for (int r = 0; r < kRounds; ++r) {
+  const int nbins = 1 << bits;
+  for (int b = tid; b < nbins; b += kSortBlock) {
+    base[b] = hist[b * nblocks + blockIdx.x];
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) wcount[w][tid] = 0;
-    __syncthreads();
+    for (int w = 0; w < kWaves; ++w) wcount[w][b] = 0;
+  }
+  __syncthreads();
+  const unsigned long long lt = (1ull << lane) - 1ull;
+  const int64_t tbase = blockIdx.x * (int64_t)(kSortBlock * rounds);
+  for (int r = 0; r < rounds; ++r) {
     const int64_t i = tbase + r * kSortBlock + tid;
     const bool valid = i < n;
     int key = 0, val = 0, digit = 0;
     if (valid) {
-      key = kin[i];
-      val = vin[i];
-      digit = (key >> shift) & 255;
+      key = load_key<FIRST>(kin, i, max_key);
+      val = FIRST ? (int)i : vin[i];
+      digit = (key >> shift) & (nbins - 1);
     }
     unsigned long long mask = __ballot(valid);
-#pragma unroll
-    for (int b = 0; b < 8; ++b) {
+    for (int b = 0; b < bits; ++b) {
       const int bit = (digit >> b) & 1;
       const unsigned long long bal = __ballot(bit);
       mask &= bit ? bal : ~bal;
     }
     const int rank = __popcll(mask & lt);
-    if (valid && rank == 0) wcount[wave][digit] = __popcll(mask);
+    if (valid && rank == 0) wcount[wave][digit] = (unsigned short)__popcll(mask);
     __syncthreads();
     if (valid) {
       int off = base[digit] + rank;
@@ -168,11 +222,17 @@ __global__ __launch_bounds__(kSortBlock) void k_rs_scatter(const int* kin, const
       kout[off] = key;
       vout[off] = val;
     }
+    if (r + 1 == rounds) break;  // the same for every thread
     __syncthreads();
-    int tot = 0;
+    for (int b = tid; b < nbins; b += kSortBlock) {
+      int tot = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) tot += wcount[w][tid];
-    base[tid] += tot;
+      for (int w = 0; w < kWaves; ++w) {
+        tot += wcount[w][b];
+        wcount[w][b] = 0;
+      }
+      base[b] += tot;
+    }
     __syncthreads();
   }
 }
@@ -180,44 +240,52 @@ __global__ __launch_bounds__(kSortBlock) void k_rs_scatter(const int* kin, const
 void radix_sort_by_cell(const int* cell, int64_t n, int max_key, int* keys_out, int* vals_out,
                         int* tmp, hipStream_t st) {
   if (n <= 0) return;
+  const int rounds = rounds_for(n);
   const int64_t nb = tiles_for(n);
-  int* k0 = tmp;
-  int* v0 = tmp + n;
-  int* k1 = tmp + 2 * n;
-  int* v1 = tmp + 3 * n;
-  int* hist = tmp + 4 * n;
-  int* tile_sums = hist + 256 * nb;
-  const int64_t ntiles = (256 * nb + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(k_rs_init, dim3((unsigned)((n + kSortBlock - 1) / kSortBlock)),
-                     dim3(kSortBlock), 0, st, cell, n, max_key, k0, v0);
+  int* hist = tmp + 2 * n;
   int bits = 1;
   while (bits < 31 && (1ll << bits) <= (long long)max_key) ++bits;
-  const int passes = (bits + 7) / 8;
-  const int* sk = k0;
-  const int* sv = v0;
+  const int passes = (bits + kMaxBits - 1) / kMaxBits;
+  const int width = (bits + passes - 1) / passes;
+  const int nbins = 1 << width;
+  const int64_t total = nbins * nb;
+  const int64_t ntiles = (total + kScanTile - 1) / kScanTile;
+  int* tile_sums = hist + total;
+  const int* sk = cell;
+  const int* sv = nullptr;
   for (int pass = 0; pass < passes; ++pass) {
-    int* dk;
-    int* dv;
-    if (pass == passes - 1) {
-      dk = keys_out;
-      dv = vals_out;
-    } else if (pass % 2 == 0) {
-      dk = k1;
-      dv = v1;
+    // the passes alternate between the outputs and tmp and end in the outputs
+    const bool out = (passes - 1 - pass) % 2 == 0;
+    int* dk = out ? keys_out : tmp;
+    int* dv = out ? vals_out : tmp + n;
+    const int shift = width * pass;
+    const dim3 g((unsigned)nb), b(kSortBlock);
+    if (pass == 0)
+      hipLaunchKernelGGL((k_rs_hist<true>), g, b, 0, st, sk, n, max_key, shift, nbins, rounds,
+                         hist, nb);
+    else
+      hipLaunchKernelGGL((k_rs_hist<false>), g, b, 0, st, sk, n, max_key, shift, nbins, rounds,
+                         hist, nb);
+    if (total <= kScanOne) {
+      hipLaunchKernelGGL(k_rs_scan_one, dim3(1), dim3(1024), 0, st, hist, (int)total);
     } else {
-      dk = k0;
-      dv = v0;
+      hipLaunchKernelGGL(k_rs_scan_tiles, dim3((unsigned)ntiles), dim3(256), 0, st, hist, total,
+                         tile_sums);
+      if (ntiles <= kScanDirect) {
+        hipLaunchKernelGGL((k_rs_scan_add<true>), dim3((unsigned)ntiles), dim3(256), 0, st, hist,
+                           total, tile_sums);
+      } else {
+        hipLaunchKernelGGL(k_rs_scan_sums, dim3(1), dim3(256), 0, st, tile_sums, ntiles);
+        hipLaunchKernelGGL((k_rs_scan_add<false>), dim3((unsigned)ntiles), dim3(256), 0, st, hist,
+                           total, tile_sums);
+      }
     }
-    const int shift = 8 * pass;
-    hipLaunchKernelGGL(k_rs_hist, dim3((unsigned)nb), dim3(kSortBlock), 0, st, sk, n, shift, hist,
-                       nb);
-    hipLaunchKernelGGL(k_rs_scan_tiles, dim3((unsigned)ntiles), dim3(256), 0, st, hist, 256 * nb,
-                       tile_sums);
-    hipLaunchKernelGGL(k_rs_scan_sums, dim3(1), dim3(256), 0, st, tile_sums, ntiles);
-    hipLaunchKernelGGL(k_rs_scan_add, dim3((unsigned)ntiles), dim3(256), 0, st, hist, 256 * nb,
-                       tile_sums);
-    hipLaunchKernelGGL(k_rs_scatter, dim3((unsigned)nb), dim3(kSortBlock), 0, st, sk, sv, dk, dv,
-                       n, shift, hist, nb);
+    if (pass == 0)
+      hipLaunchKernelGGL((k_rs_scatter<true>), g, b, 0, st, sk, sv, dk, dv, n, max_key, shift,
+                         width, rounds, hist, nb);
+    else
+      hipLaunchKernelGGL((k_rs_scatter<false>), g, b, 0, st, sk, sv, dk, dv, n, max_key, shift,
+                         width, rounds, hist, nb);
     sk = dk;
     sv = dv;
   }
