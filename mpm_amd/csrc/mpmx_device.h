@@ -300,7 +300,8 @@ MPMX_DEV void q4_natural_coordinates(const double (*X)[2], const double* pt, dou
 // a value is not a number: the caller then runs the general loop.
 // Bound by FP64 issue and by the slowest lane of a wave. 254k particles in
 // 0.01 m cells draped over a slope, locate per step: 8.55 ms with the general
-// loop, 1.6 ms with single steps of r, 0.27 ms with the powers of F.
+// loop, 1.6 ms with single steps of r, 0.27 ms with the powers of F and 0.22
+// with the general form out of line (iso_general_hex).
 MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr, double* nr_res) {
 #pragma clang fp contract(fast)
   double d[3], cx[3], cy[3], cz[3], cxy[3], cyz[3], cxz[3], cxyz[3];
@@ -544,10 +545,11 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
 // iteration matrix is jacobian_local on the unit cell's own vertices,
 // cell.tcc:772). Returns false where the reference throws (NaN).
 // FAST: hex8 cells iterate by iso_iterate_hex (the same end point to
-// rounding and 2e-13).
+// rounding and 2e-13); *general is set where that does not apply and the
+// caller has to take the general form.
 template <int D, bool FAST = false>
 MPMX_DEV bool transform_real_to_unit_cell(const double (*X)[D], double mean_length,
-                                          const double* p, double* xi) {
+                                          const double* p, double* xi, bool* general = nullptr) {
   constexpr int NN = Elem<D>::NN;
   const double big = 1.7976931348623157e308;
   double an_xi[D], an_res[D];
@@ -632,19 +634,14 @@ MPMX_DEV bool transform_real_to_unit_cell(const double (*X)[D], double mean_leng
       nr[k] = 1. - 1.E-12;
     nr_res[k] = big;
   }
-  bool done = false;
   if constexpr (D == 3 && FAST) {
-    double s[3] = {nr[0], nr[1], nr[2]}, sr[3];
-    done = iso_iterate_hex(X, p, s, sr);
-    if (done) {
+    *general = !iso_iterate_hex(X, p, nr, nr_res);
+    const bool geo = sqrt(sqnorm<D>(g_res)) < sqrt(sqnorm<D>(nr_res));
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        nr[k] = s[k];
-        nr_res[k] = sr[k];
-      }
-    }
+    for (int k = 0; k < D; ++k) xi[k] = geo ? g_xi[k] : nr[k];
+    return !(isnan(xi[0]) || isnan(xi[1]));
   }
-  for (int iter = done ? 10000 : 0; iter < 10000; ++iter) {
+  for (int iter = 0; iter < 10000; ++iter) {
     double J[D][D], Ji[D][D];
 #pragma unroll
     for (int a = 0; a < D; ++a)
@@ -722,6 +719,15 @@ MPMX_DEV bool transform_real_to_unit_cell(const double (*X)[D], double mean_leng
   return !(isnan(xi[0]) || isnan(xi[1]));
 }
 
+// The general form out of line: what it keeps in registers would spill the
+// fast one (which runs almost always).
+static __device__ __attribute__((noinline)) bool iso_general_hex(const Mesh& M, int c,
+                                                                 const double* p, double* xi) {
+  double X[8][3];
+  load_cell_X<3>(M, c, X);
+  return transform_real_to_unit_cell<3, false>(X, M.two_mean[c] * 0.5, p, xi);
+}
+
 // --------------------------- locate (cell.tcc:324-380) ----------------------
 // ISO: the mesh is isoparametric (local coordinates by
 // transform_real_to_unit_cell); else Cartesian (local_coordinates_point).
@@ -741,7 +747,14 @@ MPMX_DEV bool point_in_cell(const Mesh& M, int c, const double* p, double* xi) {
     constexpr int NN = Elem<D>::NN;
     double X[NN][D];
     load_cell_X<D>(M, c, X);
-    if (!transform_real_to_unit_cell<D, FAST>(X, M.two_mean[c] * 0.5, p, xi)) return false;
+    if constexpr (D == 3 && FAST) {
+      bool general = false;
+      bool ok = transform_real_to_unit_cell<3, true>(X, M.two_mean[c] * 0.5, p, xi, &general);
+      if (general) ok = iso_general_hex(M, c, p, xi);
+      if (!ok) return false;
+    } else {
+      if (!transform_real_to_unit_cell<D>(X, M.two_mean[c] * 0.5, p, xi)) return false;
+    }
   }
 #pragma unroll
   for (int k = 0; k < D; ++k) {

@@ -461,7 +461,7 @@ __global__ __launch_bounds__(kBlock) void k_locate_init(Mesh M, Particles P, Sta
 
 // Per-step locate of an isoparametric mesh (the step kernels locate Cartesian
 // meshes themselves): current cell, then neighbours, else the scan queue.
-// FAST: fast mode's iteration for hex8 cells (two waves per SIMD: 0.27 ms on
+// FAST: fast mode's iteration for hex8 cells (two waves per SIMD: 0.22 ms on
 // the 254k-particle draped block against 0.34 ms at one without spills).
 template <int D, bool FAST>
 __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_locate_step(Mesh M, Particles P, Status* S,
