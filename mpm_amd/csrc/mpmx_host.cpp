@@ -175,6 +175,7 @@ struct mpmx_ctx {
   DBuf<double> d_plastic_trial; // Particles::plastic_trial (any_mc_rate)
   DBuf<double> d_Cmat, d_beta;  // affine transfer matrices, ASFLIP beta (affine())
   DBuf<double> d_gterm;         // Particles::gterm (ordered mode)
+  DBuf<unsigned char> d_grank;  // Particles::grank (ordered MUSL)
   DBuf<int> d_plastic_list;     // deferred Mohr-Coulomb return mappings
   DBuf<double> d_plastic_rec;
   DBuf<Status> d_status;
@@ -298,6 +299,7 @@ struct mpmx_ctx {
     P.rotF = any_gn ? d_rotF.p : nullptr;
     P.plastic_trial = any_mc_rate ? d_plastic_trial.p : nullptr;
     P.gterm = (flags & MPMX_ORDERED) ? d_gterm.p : nullptr;
+    P.grank = (flags & MPMX_ORDERED) && scheme == MUSL ? d_grank.p : nullptr;
     P.Bmat = affine() ? d_Bmat.p : nullptr;
     P.Cmat = affine() ? d_Cmat.p : nullptr;
     P.beta = affine() ? d_beta.p : nullptr;
@@ -914,6 +916,7 @@ void alloc_step_buffers(mpmx_ctx* c) {
     c->d_cstart.alloc(std::max<int64_t>(c->ncells, 1));
     c->d_cend.alloc(std::max<int64_t>(c->ncells, 1));
     c->d_gterm.alloc((size_t)c->nn * (1 + c->dim) * std::max<int64_t>(np, 1));
+    if (c->scheme == MUSL) c->d_grank.alloc((size_t)c->nn * std::max<int64_t>(np, 1));
   }
 }
 
@@ -1109,6 +1112,7 @@ struct StepBuffers {
   double* rotF;   // Green-Naghdi scratch; rotated trial stresses of the deferred list
   double* plastic_trial;
   double* gterm;  // ordered mode: per-particle gather terms
+  unsigned char* grank = nullptr;  // ordered MUSL: the gathers' ranks
   Status* host = nullptr;  // pinned memory that takes the status at the step's end
 };
 
@@ -1130,6 +1134,7 @@ StepBuffers ctx_buffers(mpmx_ctx* c) {
   B.rotF = c->d_rotF.p;
   B.plastic_trial = c->d_plastic_trial.p;
   B.gterm = c->d_gterm.p;
+  B.grank = c->d_grank.p;
   return B;
 }
 
@@ -1200,6 +1205,7 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
   if (P.rotF) P.rotF = B.rotF;
   if (P.plastic_trial) P.plastic_trial = B.plastic_trial;
   if (P.gterm) P.gterm = B.gterm;
+  P.grank = P.grank ? B.grank : nullptr;
   Nodes Nd = c->nodes();
   if (Nd.fnval) Nd.fnval = B.fnval;
   hipStream_t st = c->stream;

@@ -160,6 +160,10 @@ struct Particles {
   // -(dN_i/dx . sigma)_k V), written before a force gather (null in fast
   // mode).
   double* gterm;
+  // Ordered MUSL: [NN][np] each particle's rank among the particles of each
+  // node of its cell, from the force gather to the momentum gather of the step
+  // (null: ranked again)
+  unsigned char* grank;
   int* plastic_list;
   double* plastic_rec;  // [PR_N][np] by list slot
   // Particle tractions (Particle::assign_traction / map_traction_force,

@@ -1800,7 +1800,11 @@ __global__ void k_clear_pair(int* a, int* b, int64_t n) {
 // contributions and stores them at their rank in LDS; then one lane per
 // sum folds it in rank order, so every sum adds the same terms in the same
 // order as one thread walking the particles by id. A node with more than
-// kGatherMax particles is summed by one lane merging the cell lists.
+// kGatherMax particles is summed by one lane merging the cell lists. The terms
+// pass through LDS 64 ranks at a time: a node of a full grid has 64 (3D) and
+// the waves in flight are what hides the gathers' latency (262k particles,
+// force gather with its preparation: 145 us with 128 slots, 128 now; MUSL's
+// momentum gather 63 us ranking again, 53 with the force gather's ranks).
 constexpr int kGatherMax = 128;
 
 // Slots of a node's sums: mass, momentum, external force, internal force.
@@ -1916,16 +1920,26 @@ MPMX_DEV void gather_terms(const Mesh& M, const Particles& P, int64_t n, int p, 
   }
 }
 
+// Waves per SIMD of the gathers: the 3D sums of all quantities gain from 5 (128
+// us against 132) and MUSL's second momentum, which takes its ranks ready-made,
+// from 7, as do the 2D ones (16.0 us against 17.8 at 6400 particles); USF's
+// two 3D ones are best as the compiler has them (262k particles:
+// 74 / 105 us, at 5 waves 83 / 120).
+template <int D, int WHAT>
+constexpr int gather_waves() {
+  return D == 2 || WHAT == SC_MOM ? 7 : WHAT == (SC_MV | SC_F) ? 5 : 1;
+}
+
 template <int D, int WHAT, int FL>
-__global__ __launch_bounds__(64) void k_gather(Mesh M, Particles P, Nodes Nd, StepArgs A,
-                                               const Status* S, const int* perm,
-                                               const int* cstart, const int* cend) {
+__global__ __launch_bounds__(64) MPMX_WAVES((gather_waves<D, WHAT>())) void k_gather(
+    Mesh M, Particles P, Nodes Nd, StepArgs A, const Status* S, const int* perm,
+    const int* cstart, const int* cend) {
   if (run_stopped(S)) return;
   using GS = GatherSlots<D>;
   constexpr int NN = Elem<D>::NN;
   constexpr int NV = GS::N;
   constexpr int V0 = GS::template first<WHAT>(), NU = GS::template count<WHAT>();
-  __shared__ double terms[NU][kGatherMax];  // the used slots V0 .. V0 + NU - 1
+  __shared__ double terms[NU][64];  // 64 ranks of the used slots V0 .. V0 + NU - 1
   const int lane = threadIdx.x;
   const int64_t n = blockIdx.x;
   if (n >= M.nnodes) return;
@@ -1993,45 +2007,64 @@ __global__ __launch_bounds__(64) void k_gather(Mesh M, Particles P, Nodes Nd, St
     // (stable sort of id-ordered input) and the lists are disjoint, so a
     // particle's rank is the sum over the lists of how many of their ids are
     // below its own (its own list: its position there), each count by a
-    // binary search in LDS with the list's (wave-uniform) power-of-two steps
-    __shared__ int ids[kGatherMax];
-#pragma unroll
-    for (int q = 0; q < 2; ++q)
-      if (lane + 64 * q < T) ids[lane + 64 * q] = ps[q];
-    __syncthreads();
+    // binary search in LDS with the list's (wave-uniform) power-of-two steps.
+    // The force gather leaves the ranks for MUSL's momentum gather of the step.
     const int nq = T > 64 ? 2 : 1;
     int rk[2] = {0, 0};
+    if (WHAT == SC_MOM && P.grank) {
 #pragma unroll
-    for (int j = 0; j < NN; ++j) {
-      const int len = (j + 1 < NN ? off[j + 1] : T) - off[j];
-      if (len == 0) continue;
-      const int top = 1 << (31 - __builtin_clz(len));  // largest power of two <= len
+      for (int q = 0; q < 2; ++q)
+        if (lane + 64 * q < T) rk[q] = P.grank[(int64_t)is[q] * np + ps[q]];
+    } else {
+      __shared__ int ids[kGatherMax];
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (lane + 64 * q < T) ids[lane + 64 * q] = ps[q];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < NN; ++j) {
+        const int len = (j + 1 < NN ? off[j + 1] : T) - off[j];
+        if (len == 0) continue;
+        const int top = 1 << (31 - __builtin_clz(len));  // largest power of two <= len
 #pragma unroll 1
-      for (int q = 0; q < nq; ++q) {
-        const int a = q ? ps[1] : ps[0];
-        int below = 0;
-        for (int step = top; step > 0; step >>= 1)
-          if (below + step <= len && ids[off[j] + below + step - 1] < a) below += step;
-        if (q) rk[1] += below;
-        else rk[0] += below;
+        for (int q = 0; q < nq; ++q) {
+          const int a = q ? ps[1] : ps[0];
+          int below = 0;
+          for (int step = top; step > 0; step >>= 1)
+            if (below + step <= len && ids[off[j] + below + step - 1] < a) below += step;
+          if (q) rk[1] += below;
+          else rk[0] += below;
+        }
+      }
+      if (WHAT == (SC_MV | SC_F) && P.grank) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          if (lane + 64 * q < T) P.grank[(int64_t)is[q] * np + ps[q]] = (unsigned char)rk[q];
       }
     }
-#pragma unroll 1
-    for (int q = 0; q < 2; ++q) {  // one slot at a time (register pressure)
-      if (lane + 64 * q < T) {
-        const int pq = q ? ps[1] : ps[0], iq = q ? is[1] : is[0];
-        const int rq = q ? rk[1] : rk[0];
-        double out[NV];
-        gather_terms<D, WHAT>(M, P, n, pq, iq, g, out);
-#pragma unroll
-        for (int v = 0; v < NU; ++v) terms[v][rq] = out[V0 + v];
-      }
-    }
-    __syncthreads();
+    // 64 ranks at a time: the terms of the particles ranked there, then the
+    // fold goes on in rank order
     double acc = 0.;
-    if (lane < NU) {
+#pragma unroll 1
+    for (int w = 0; w < T; w += 64) {
+      if (w > 0) __syncthreads();  // the ranks before are folded
+#pragma unroll 1
+      for (int q = 0; q < nq; ++q) {  // one slot at a time (register pressure)
+        const int rq = (q ? rk[1] : rk[0]) - w;
+        if (lane + 64 * q < T && rq >= 0 && rq < 64) {
+          const int pq = q ? ps[1] : ps[0], iq = q ? is[1] : is[0];
+          double out[NV];
+          gather_terms<D, WHAT>(M, P, n, pq, iq, g, out);
+#pragma unroll
+          for (int v = 0; v < NU; ++v) terms[v][rq] = out[V0 + v];
+        }
+      }
+      __syncthreads();
+      if (lane < NU) {
+        const int m = T - w < 64 ? T - w : 64;
 #pragma unroll 8
-      for (int r = 0; r < T; ++r) acc = acc + terms[lane][r];
+        for (int r = 0; r < m; ++r) acc = acc + terms[lane][r];
+      }
     }
 #pragma unroll
     for (int v = 0; v < NU; ++v) sums[V0 + v] = __shfl(acc, v, 64);
