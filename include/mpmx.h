@@ -57,8 +57,8 @@ typedef struct mpmx_ctx mpmx_ctx;
 /* creation flags */
 #define MPMX_ORDERED 0x1u /* nodal sums in particle order: bitwise equal to a
                              single-threaded reference run (slower) */
-#define MPMX_NO_GRAPH 0x2u /* launch kernels directly instead of replaying a
-                              captured hipGraph per step */
+#define MPMX_NO_GRAPH 0x2u /* launch kernels directly, also in long runs of
+                              steps (else replayed from captured hipGraphs) */
 
 /* Number of doubles in one material parameter vector (layout documented in
  * mpm_amd/materials.py; replaces Factory<Material<Tdim>, unsigned, const Json&>
