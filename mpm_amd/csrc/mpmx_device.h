@@ -295,7 +295,8 @@ MPMX_DEV void q4_natural_coordinates(const double (*X)[2], const double* pt, dou
 //    (e = xi - x*). Powers F^(2^j) to second order take the steps up to a few
 //    before the last at once; the last ones, which decide where the iteration
 //    stops, are single steps. Used from where the neglected third order moves
-//    the end point by less than 2e-13.
+//    the end point by less than 2e-13, and only where each step taken so is
+//    known to decrease the residual (else the line search would act on it).
 // Returns false where a step does not decrease the residual (line search) or
 // a value is not a number: the caller then runs the general loop.
 // Bound by FP64 issue and by the slowest lane of a wave. 254k particles in
@@ -384,7 +385,32 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
                  c = cxz[k] + xs[1] * cxyz[k];
     q2 = q2 + ((a * a + b * b) + (c * c + cxyz[k] * cxyz[k]));
   }
-  const double bend = sqrt(q2) * inv;
+  const double turn = sqrt(q2), bend = turn * inv;
+  // A step decreases the residual, |(I - M') r| < |r|, if M' + M'^T - M'^T M' is
+  // positive definite for its mean Jacobian M', which lies within 2 turn |e|
+  // of M: so it is while |e| <= reach.
+  float reach = 0.f;  // in 32 bits: an error of 1e-6 against a slack of 1 / 64
+  if (solved) {
+    double M[3][3];
+    jacobian(xs, M);
+    float m[3][3], S[3][3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b < 3; ++b) m[a][b] = (float)M[a][b];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int b = 0; b <= a; ++b)
+        S[a][b] = (m[a][b] + m[b][a]) - (m[0][a] * m[0][b] + m[1][a] * m[1][b] + m[2][a] * m[2][b]);
+    const float slack = 0.015625f * fminf(S[0][0], fminf(S[1][1], S[2][2]));
+#pragma unroll
+    for (int a = 0; a < 3; ++a) S[a][a] = S[a][a] - slack;
+    const float m2 = S[0][0] * S[1][1] - S[1][0] * S[1][0];
+    const float m3 = S[2][2] * m2 - S[2][0] * (S[2][0] * S[1][1] - S[2][1] * S[1][0]) -
+                     S[2][1] * (S[0][0] * S[2][1] - S[1][0] * S[2][0]);
+    if (slack > 0.f && m2 > 0.f && m3 > 0.f) reach = slack / (4.f * (float)turn);
+  }
   int it = 0, jumps = 0;
   while (it < 10000) {
     if (solved && (it & 15) == 0 && n2 > 4. * kTol2) {
@@ -398,7 +424,7 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
       // by at least sqrt(ef / |e|) (modes that fade at different rates), ef =
       // 1e-10 |e| / |r|
       const double en = sqrt(e2), rn = sqrt(n2);
-      if ((bend * en) * (bend * en + en) * en * sqrt(1e-10 / rn) < 2e-13) {
+      if ((bend * en) * (bend * en + en) * en * sqrt(1e-10 / rn) < 2e-13 && en <= reach) {
         // steps of the linear part until |A^n r| < 1e-10 (M commutes with
         // A = I - M): bracketed by powers of two, then by the rate of the last
         // octave before; modes fade at different rates and the rate only
