@@ -302,7 +302,10 @@ MPMX_DEV void q4_natural_coordinates(const double (*X)[2], const double* pt, dou
 // Bound by FP64 issue and by the slowest lane of a wave. 254k particles in
 // 0.01 m cells draped over a slope, locate per step: 8.55 ms with the general
 // loop, 1.6 ms with single steps of r, 0.27 ms with the powers of F and 0.22
-// with the general form out of line (iso_general_hex).
+// with the general form out of line (iso_general_hex). In cells of 1 mm and
+// less the iteration's limit comes first; jumped to as well, 188k particles in
+// cells of 0.5 and 1 mm take 0.08 ms (8.6 ms where such jumps were refused and
+// sought again every 16 steps).
 MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr, double* nr_res) {
 #pragma clang fp contract(fast)
   double d[3], cx[3], cy[3], cz[3], cxy[3], cyz[3], cxz[3], cxyz[3];
@@ -342,6 +345,7 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
     }
   };
   constexpr double kTol2 = 1e-20;  // (1e-10)^2
+  constexpr int kMaxIter = 10000;
   double r[3];
   double n2 = residual(nr, r);
   // x*: 3 to 5 steps on a cell that is not degenerate; without convergence
@@ -411,8 +415,9 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
                      S[2][1] * (S[0][0] * S[2][1] - S[1][0] * S[2][0]);
     if (slack > 0.f && m2 > 0.f && m3 > 0.f) reach = slack / (4.f * (float)turn);
   }
-  int it = 0, jumps = 0;
-  while (it < 10000) {
+  // a point makes at most 3 jumps, or 12 tries
+  int it = 0, tries = 0;
+  while (it < kMaxIter) {
     if (solved && (it & 15) == 0 && n2 > 4. * kTol2) {
       double e[3], e2 = 0.;
 #pragma unroll
@@ -430,6 +435,7 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
         // octave before; modes fade at different rates and the rate only
         // falls, so this stops short (a later jump takes up what is left)
         int n = 0;
+        const int left = kMaxIter - 32 - it;  // to just before the iteration's limit
         double M[3][3];
         jacobian(xs, M);
         {
@@ -440,7 +446,7 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
             for (int c = 0; c < 3; ++c) P[k][c] = (k == c ? 1. : 0.) - M[k][c];
           float la = 0.f, lb = __log2f((float)n2);
 #pragma unroll 1
-          for (int len = 1; len <= 8192; len *= 2) {
+          for (int len = 1; len <= left; len *= 2) {
             double s2 = 0., Q[3][3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -462,11 +468,14 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
           // la: at n / 2 steps (n = 1: at the start); -66.4 = log2(kTol2)
           const float more = (lb + 66.43856f) * (n > 1 ? 0.5f * n : 1.f) / (la - lb);
           n += (int)fminf(fmaxf(more, 0.f), (float)n);
+          if (n > left)  // the limit comes first, and the third order may not have faded
+            n = (bend * en) * (bend * en + en) * en < 2e-13 ? left : 0;
         }
         // stop short of it: the second order shifts the count by about
         // bend |e| / (rate of decrease)
         n -= 4 + (int)fmin(1e4, 2. * bend * en * inv);
-        if (n >= 24 && it + n < 9000) {
+        tries += 1;
+        if (n >= 24) {
           // F^n by its binary digits; B: monomials xx, yy, zz, xy, yz, xz
           double P[3][3], B[3][6];
 #pragma unroll
@@ -539,8 +548,9 @@ MPMX_DEV bool iso_iterate_hex(const double (*X)[3], const double* p, double* nr,
             n2 = t2;
             it += n;
           }
-          if (++jumps == 3) solved = false;
+          tries += 3;
         }
+        if (tries >= 12) solved = false;
       }
     }
     double t[3], tr[3];

@@ -44,3 +44,14 @@ def test_fast_inverse_is_the_general_loops(check, h, distortion, seed, points):
     assert n > points // 2
     assert differing == 0
     assert worst <= 2e-10, worst
+
+
+# A search for the number of steps to jump is up to 14 squarings of the step's
+# matrix. Cells of some mm reach the loop's limit of 10000 steps first: 12
+# searches of up to 15 octaves a point, not one every 16 steps.
+@pytest.mark.parametrize("h", [0.0005, 0.001, 0.002, 0.003, 0.005])
+@pytest.mark.parametrize("distortion", [0.02, 0.1, 0.4, 0.6])
+def test_refused_jumps_are_not_sought_again_and_again(check, h, distortion):
+    n, general, differing, worst, octaves = check(1, 300, h, distortion)
+    assert differing == 0 and worst <= 2e-10
+    assert octaves <= 12 * 15, octaves
