@@ -230,6 +230,7 @@ struct mpmx_ctx {
   DBuf<char> d_read;
   char* h_read = nullptr;  // pinned
   size_t read_bytes = 0;   // of each of the two halves
+  bool was_read = false;
   hipEvent_t read_done[2] = {nullptr, nullptr};
 
   // profiling
@@ -755,16 +756,56 @@ struct ReadField {
   int comps, kind, size;
 };
 
+// The array's components one by one, transposed on the host.
+template <class T, class R>
+void read_components(const ReadField& f, int64_t n, hipStream_t st) {
+  std::vector<T> col(n);
+  R* rows = (R*)f.out;
+  for (int k = 0; k < f.comps; ++k) {
+    HIPCHECK(hipMemcpyAsync(col.data(), (const T*)f.in + (size_t)k * n, n * sizeof(T),
+                            hipMemcpyDeviceToHost, st));
+    HIPCHECK(hipStreamSynchronize(st));
+    for (int64_t i = 0; i < n; ++i) rows[i * f.comps + k] = col[i];
+  }
+}
+
 // Copies fields of n particles to the host: packed into rows by a kernel, a
 // piece of the staging at a time, each piece one copy to pinned memory while
 // the piece before it is spread to the caller's arrays. (A copy per component
 // and a transposition on the host took 0.5 ms for 8192 particles, most of it
 // the 63 copies' latency.) The staging, twice the size of the largest read so
 // far and at most 2 x 4 MiB on each side, stays the context's.
+// A context's first read makes the staging, up to 2 ms of fresh pinned pages.
+// Where that is more than the first read gains, which may be the only one, the
+// components are copied one by one: few of them, and neither so little data
+// that the staging costs nothing nor so much that one read pays for it. x and
+// v, first read with copies / with the staging made / later reads: 512
+// particles 93 / 67 / 24 us, 8192 67 / 86 / 49, 24k 110 / 145 / 75, 111k 410 /
+// 455 to 2400 / 270, 262k (3D) 1800 / 980 to 4400 / 740, 2M (3D) 16400 / 9900 /
+// 6200; all 63 components of 8192 particles 660 / 270 / 200.
+constexpr int kFirstReadCopies = 8;
+constexpr size_t kFirstReadMin = size_t(128) << 10, kFirstReadMax = size_t(32) << 20;
 void read_rows(mpmx_ctx* c, const std::vector<ReadField>& f, int64_t n) {
   if (f.empty()) return;
   size_t want = size_t(64) << 10, total = 0;
-  for (const auto& q : f) total += (size_t)q.comps * q.size * n + 16;
+  int copies = 0;
+  for (const auto& q : f) {
+    total += (size_t)q.comps * q.size * n + 16;
+    copies += q.comps;
+  }
+  const bool first = !c->was_read;
+  c->was_read = true;
+  if (first && copies <= kFirstReadCopies && total >= kFirstReadMin && total <= kFirstReadMax) {
+    for (const auto& q : f) {
+      if (q.kind == PACK_F64)
+        read_components<double, double>(q, n, c->stream);
+      else if (q.kind == PACK_I32)
+        read_components<int, int>(q, n, c->stream);
+      else
+        read_components<int, int64_t>(q, n, c->stream);
+    }
+    return;
+  }
   while (want < total && want < (size_t(4) << 20)) want *= 2;
   if (c->read_bytes < want) {
     if (c->h_read) (void)hipHostFree(c->h_read);
