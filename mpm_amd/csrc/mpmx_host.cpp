@@ -176,7 +176,7 @@ struct mpmx_ctx {
   DBuf<double> d_Cmat, d_beta;  // affine transfer matrices, ASFLIP beta (affine())
   DBuf<double> d_gterm;         // Particles::gterm (ordered mode)
   DBuf<unsigned char> d_grank;  // Particles::grank (ordered MUSL)
-  DBuf<int> d_plastic_list;     // deferred Mohr-Coulomb return mappings
+  DBuf<int> d_plastic_list;     // deferred Mohr-Coulomb return mappings (defers_plastic())
   DBuf<double> d_plastic_rec;
   DBuf<Status> d_status;
   Status* h_status = nullptr;  // pinned
@@ -304,7 +304,7 @@ struct mpmx_ctx {
     P.Bmat = affine() ? d_Bmat.p : nullptr;
     P.Cmat = affine() ? d_Cmat.p : nullptr;
     P.beta = affine() ? d_beta.p : nullptr;
-    P.plastic_list = any_mc ? d_plastic_list.p : nullptr;
+    P.plastic_list = any_mc ? d_plastic_list.p : nullptr;  // null where nothing is deferred
     P.plastic_rec = any_mc ? d_plastic_rec.p : nullptr;
     P.ntr = ntr;
     P.tr_list = ntr ? d_tr_list.p : nullptr;
@@ -934,6 +934,22 @@ double particle_size(double volume, int dim) {
   return std::pow(volume, static_cast<double>(1. / dim));
 }
 
+// Whether the stress kernels use fast mode's regrouped arithmetic
+// (mpmx_fast.h): in 3D without a stress rate. There fast mode's nodal sums
+// (four and more atomic contributions per node) already differ from run to
+// run by rounding, which a plastic run magnifies, and 10 + 10 steps of the
+// 2.1M-particle collapse differ as much between two runs of one build as
+// between the two arithmetics (velocities 1e-13 to 6e-9 over seeds). In 2D a
+// node has two contributions as a rule, runs repeat to 1e-12, and the
+// reference's arithmetic is kept.
+bool fast_stress(const mpmx_ctx* c) {
+  return c->dim == 3 && !(c->flags & MPMX_ORDERED) && !c->any_rate;
+}
+
+// Whether the step's kernels defer yielding particles to k_plastic (3D fast mode
+// without a stress rate returns them in the stress kernels).
+bool defers_plastic(const mpmx_ctx* c) { return c->any_mc && !fast_stress(c); }
+
 void alloc_step_buffers(mpmx_ctx* c) {
   const int64_t np = c->np;
   c->d_skey.alloc(std::max<int64_t>(np, 1));
@@ -948,7 +964,7 @@ void alloc_step_buffers(mpmx_ctx* c) {
       c->d_Cmat.alloc((size_t)c->dim * c->dim * std::max<int64_t>(np, 1));
     c->d_beta.alloc(std::max<int64_t>(np, 1));
   }
-  if (c->any_mc) {
+  if (defers_plastic(c)) {
     c->d_plastic_list.alloc(std::max<int64_t>(np, 1));
     c->d_plastic_rec.alloc(PR_N * std::max<int64_t>(np, 1));
   }
@@ -1217,18 +1233,6 @@ struct Launcher {
   }
 };
 
-// Whether the stress kernels use fast mode's regrouped arithmetic
-// (mpmx_fast.h): in 3D without a stress rate. There fast mode's nodal sums
-// (four and more atomic contributions per node) already differ from run to
-// run by rounding, which a plastic run magnifies, and 10 + 10 steps of the
-// 2.1M-particle collapse differ as much between two runs of one build as
-// between the two arithmetics (velocities 1e-13 to 6e-9 over seeds). In 2D a
-// node has two contributions as a rule, runs repeat to 1e-12, and the
-// reference's arithmetic is kept.
-bool fast_stress(const mpmx_ctx* c) {
-  return c->dim == 3 && !(c->flags & MPMX_ORDERED) && !c->any_rate;
-}
-
 template <int D>
 void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
                   const StepBuffers& B) {
@@ -1264,10 +1268,9 @@ void enqueue_step(mpmx_ctx* c, const StepArgs& A, Launcher& L, bool full_sort,
       launch_fn_eval(c->d_fns.p, c->d_fn_data.p, (int)c->fns.size(), S, A.dt, B.fnval, st);
     });
   // the Mohr-Coulomb return mappings deferred by the stress kernels
-  // (3D fast mode without a stress rate completes them in its own kernels)
   const bool own = fast_stress(c);
   auto plastic = [&] {
-    if (c->any_mc && !own) L("mc_plastic", [&] { launch_plastic(P, mats, S, st); });
+    if (defers_plastic(c)) L("mc_plastic", [&] { launch_plastic(P, mats, S, st); });
   };
   // affine velocity updates (APIC, ASFLIP, TPIC): ordered mode's transfer
   // matrix before each gather; the mapping matrix before a G2P with stress
@@ -1592,7 +1595,7 @@ size_t carve_step_buffers(const mpmx_ctx* c, uintptr_t base, StepBuffers* B) {
   }
   B->plastic_list = nullptr;
   B->plastic_rec = nullptr;
-  if (c->any_mc) {
+  if (defers_plastic(c)) {
     B->plastic_list = (int*)take(np * sizeof(int));
     B->plastic_rec = (double*)take((size_t)PR_N * np * sizeof(double));
   }

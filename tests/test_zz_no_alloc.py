@@ -98,3 +98,16 @@ def test_noalloc_refuses_remove_mode_and_oversize():
         s.step_noalloc(1, 1e-5)
     assert e.value.code == E_ARG and "scratch" in str(e.value)
     s.step(1, 1e-5)  # the allocating entry point still runs it
+
+
+def test_noalloc_3d_fast_above_the_deferred_lists_size():
+    """512,000 Mohr-Coulomb particles: with the 116 bytes a particle of the
+    deferred list the scratch would not hold them, and 3D fast mode defers
+    nothing."""
+    w = workloads.collapse_3d(nx=48, ny=42, nz=42, block=(40, 40, 40))
+    print("noalloc 3d fast", flush=True)
+    a, b, pa, pb = _run_pair(w, False, 2)
+    assert a.nparticles == 512000
+    assert np.array_equal(pa["cell"], pb["cell"])
+    for f in ("x", "v", "stress", "strain", "F"):
+        assert _relerr(pa[f], pb[f]) <= 1e-11, f
