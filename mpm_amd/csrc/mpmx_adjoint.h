@@ -76,7 +76,7 @@ struct AdjList {
   int* ids;
   int* apex;
   double* buf;  // [6][cap]
-  double* out;  // [12][cap]
+  double* out;  // [12][cap], between k_ad_mc and its tail only
   int64_t cap;
 };
 

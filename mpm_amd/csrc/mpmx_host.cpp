@@ -1784,6 +1784,12 @@ void ad_check_supported(mpmx_ctx* c) {
   }
 }
 
+// Where the backward pass keeps the 12 output columns of its plastic list: in
+// the forward step's records of deferred returns, which hold nothing between
+// steps, or, where the forward step defers none, in columns of its own.
+static_assert(PR_N >= 12, "the records hold the adjoint list's outputs");
+bool ad_list_own_out(const mpmx_ctx* c) { return c->any_mc && !defers_plastic(c); }
+
 void ad_backward_step(mpmx_ctx* c, int j, int64_t t) {
   AdjArgs a;
   a.dt = c->ad_dt;
@@ -1804,7 +1810,7 @@ void ad_backward_step(mpmx_ctx* c, int j, int64_t t) {
   Q.ids = c->d_ad_list.p + 2;
   Q.apex = c->d_ad_list.p + 2 + c->np;
   Q.buf = c->d_ad_list_buf.p;
-  Q.out = c->d_ad_list_buf.p + 6 * c->np;
+  Q.out = ad_list_own_out(c) ? c->d_ad_list_buf.p + 6 * c->np : c->d_plastic_rec.p;
   if (c->dim == 2)
     launch_ad_backward_step<2>(c->scheme, c->mesh(), c->parts(), c->nodes(), c->d_mats.p, s0, s1,
                                ad_nodes(c, j), ad_parts(c), Q, a, c->stream);
@@ -2785,7 +2791,7 @@ void adjoint_backward(mpmx_ctx* c, bool dev, const double* dL_dx, const double* 
   c->d_ad_nodes.alloc(ad_node_doubles(c));
   c->d_ad_parts.alloc(ad_part_doubles(c));
   c->d_ad_list.alloc(2 + 2 * (size_t)np);
-  c->d_ad_list_buf.alloc(18 * (size_t)np);
+  c->d_ad_list_buf.alloc((ad_list_own_out(c) ? 18 : 6) * (size_t)np);
   launch_ad_fill(c->d_ad_parts.p, ad_part_doubles(c), 0., st);
   const AdjParticles L = ad_parts(c);
   auto put_rows = [&](double* soa, int comps, const double* rows) {

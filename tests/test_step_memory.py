@@ -40,3 +40,27 @@ assert any("k_stress_fast" in l for l in log())
 print("ok")
 """)
     assert "ok" in out
+
+
+def test_backward_pass_holds_no_more_for_its_plastic_list(lib):
+    """The backward pass's list: ids, apex flags and 6 columns a particle; its
+    12 output columns lie in the forward step's records of deferred returns,
+    or, in 3D fast mode, which has no such records, in columns of their own
+    (fewer than those records' 14)."""
+    out = hip_record.run(lib, """
+n = 4096
+for dim, ordered, mc, cols in ((2, False, True, 6), (2, True, True, 6), (3, True, True, 6),
+                               (3, False, True, 18), (3, False, False, 6)):
+    s = solver(dim, "musl", n, mc=mc, ordered=ordered)
+    s.adjoint_forward(4, 1e-6, checkpoint_every=2)
+    log()
+    p0 = rec.hip_record_device_bytes()
+    s.adjoint_backward(dL_dx=np.ones((n, dim)))
+    nodes = (2 + 8 * dim) * s.nnodes * 8
+    parts = (3 * dim + 10) * n * 8
+    held = rec.hip_record_device_bytes() - p0 - nodes - parts - (2 + 2 * n) * 4
+    assert held == cols * n * 8, (dim, ordered, held / n / 8)
+    s.close()
+print("ok")
+""")
+    assert "ok" in out
