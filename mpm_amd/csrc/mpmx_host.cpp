@@ -954,7 +954,7 @@ void alloc_step_buffers(mpmx_ctx* c) {
   const int64_t np = c->np;
   c->d_skey.alloc(std::max<int64_t>(np, 1));
   c->d_perm.alloc(std::max<int64_t>(np, 1));
-  c->d_sort_tmp.alloc(radix_sort_temp_ints(std::max<int64_t>(np, 1)));
+  c->d_sort_tmp.alloc(radix_sort_temp_ints(std::max<int64_t>(np, 1), (int)c->ncells));
   c->d_scan_list.alloc(std::max<int64_t>(np, 1));
   if (c->any_rate) c->d_spin.alloc(3 * std::max<int64_t>(np, 1));
   if (c->any_gn) c->d_rotF.alloc((size_t)(c->dim * 3 + c->dim * c->dim) * std::max<int64_t>(np, 1));
@@ -1584,7 +1584,7 @@ size_t carve_step_buffers(const mpmx_ctx* c, uintptr_t base, StepBuffers* B) {
   B->S = c->d_status.p;
   B->skey = (int*)take(np * sizeof(int));
   B->perm = (int*)take(np * sizeof(int));
-  B->sort_tmp = (int*)take(radix_sort_temp_ints(np) * sizeof(int));
+  B->sort_tmp = (int*)take(radix_sort_temp_ints(np, (int)c->ncells) * sizeof(int));
   B->scan = (int*)take(np * sizeof(int));
   B->cstart = B->cend = nullptr;
   B->gterm = nullptr;

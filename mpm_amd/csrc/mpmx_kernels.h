@@ -118,8 +118,8 @@ void take_rows(const T* in, T* out, const int* idx, int64_t nnew, int64_t nold, 
 // Stable LSD radix sort of (cell key, particle id) pairs. keys_in: cell of
 // each particle in particle order (values are the particle ids 0..n-1).
 // Sorted keys/values end in keys_out/vals_out. Temporary buffers are sized by
-// radix_sort_temp_ints(n).
-int64_t radix_sort_temp_ints(int64_t n);
+// radix_sort_temp_ints(n, max_key).
+int64_t radix_sort_temp_ints(int64_t n, int max_key);
 void radix_sort_by_cell(const int* cell, int64_t n, int max_key, int* keys_out, int* vals_out,
                         int* tmp, hipStream_t st);
 }  // namespace mpmx

@@ -45,9 +45,20 @@ static inline int64_t tiles_for(int64_t n) {
   return (n + t - 1) / t;
 }
 
-int64_t radix_sort_temp_ints(int64_t n) {
-  const int64_t nb = std::max<int64_t>(tiles_for(n), 1);
-  return 2 * n + kMaxBins * nb + (kMaxBins * nb + kScanTile - 1) / kScanTile + 64;
+// Passes and the bits of a pass's digit for keys up to max_key.
+struct Digits {
+  int passes, width;
+};
+static inline Digits digits_for(int max_key) {
+  int bits = 1;
+  while (bits < 31 && (1ll << bits) <= (long long)max_key) ++bits;
+  const int passes = (bits + kMaxBits - 1) / kMaxBits;
+  return {passes, (bits + passes - 1) / passes};
+}
+
+int64_t radix_sort_temp_ints(int64_t n, int max_key) {
+  const int64_t table = std::max<int64_t>(tiles_for(n), 1) << digits_for(max_key).width;
+  return 2 * n + table + (table + kScanTile - 1) / kScanTile + 64;
 }
 
 // keys: cell in [0, ncells) else max_key
@@ -243,10 +254,7 @@ void radix_sort_by_cell(const int* cell, int64_t n, int max_key, int* keys_out, 
   const int rounds = rounds_for(n);
   const int64_t nb = tiles_for(n);
   int* hist = tmp + 2 * n;
-  int bits = 1;
-  while (bits < 31 && (1ll << bits) <= (long long)max_key) ++bits;
-  const int passes = (bits + kMaxBits - 1) / kMaxBits;
-  const int width = (bits + passes - 1) / passes;
+  const auto [passes, width] = digits_for(max_key);
   const int nbins = 1 << width;
   const int64_t total = nbins * nb;
   const int64_t ntiles = (total + kScanTile - 1) / kScanTile;
