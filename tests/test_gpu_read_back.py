@@ -1,6 +1,6 @@
 """Reading particle state back in pieces: every field equals what was set, for
 counts around the piece boundaries (the staging holds 4 MiB: a read of all
-fields of a few thousand particles is one piece, of 100k some dozens), and any
+fields of a few thousand particles is one piece, of 100k nine), and any
 subset of fields."""
 import numpy as np
 import pytest
