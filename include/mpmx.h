@@ -331,9 +331,9 @@ int mpmx_set_particle_ids(mpmx_ctx* ctx, int64_t n, const int64_t* ids);
  * reference. */
 int mpmx_set_chunk(mpmx_ctx* ctx, int particles_per_workgroup);
 
-/* Fast mode: time trial_steps steps (after one warm-up step) for every pair
- * of scatter chunk {128, 256, 512} and full-sort interval {4, 8, 16} from the
- * current state, keep the fastest pair and restore the state (particles and
+/* Fast mode: time trial_steps steps, as a long run launches them (after a
+ * warm-up of up to 8 that instantiates its graphs), for every pair of scatter
+ * chunk {128, 256, 512} and full-sort interval {4, 8, 16} from the current state, keep the fastest pair and restore the state (particles and
  * step counter are as before the call). Writes the chosen pair. Ordered mode
  * has nothing to tune and returns the current settings. No counterpart in
  * the reference. */

@@ -2630,16 +2630,22 @@ int mpmx_autotune(mpmx_ctx* c, double dt, double damping_factor, int trial_steps
     try {
       for (const int ch : {128, 256, 512})
         for (const int se : {4, 8, 16}) {
-          copy_state(false);
-          c->step = step0;
           c->chunk = ch;
           c->sort_every = se;
-          c->need_sort = true;
           c->invalidate_graph();
-          reset_status(c);
-          launch_steps(c, 1, dt, damping_factor);  // capture, first sort
-          HIPCHECK(hipEventRecord(e0, c->stream));
-          launch_steps(c, trial_steps, dt, damping_factor);
+          // a run's steady state: the graphs instantiated (the blocks with and
+          // without a sort) before the timed steps, which begin with a sort
+          c->graph_steps = kGraphAfter;
+          c->graph_dt = dt;
+          c->graph_damping = damping_factor;
+          for (const int steps : {std::min(trial_steps, 2 * kBlockSteps), trial_steps}) {
+            copy_state(false);
+            c->step = step0;
+            c->need_sort = true;
+            reset_status(c);
+            HIPCHECK(hipEventRecord(e0, c->stream));
+            launch_steps(c, steps, dt, damping_factor);
+          }
           HIPCHECK(hipEventRecord(e1, c->stream));
           check_status(c);
           float ms = 0.f;

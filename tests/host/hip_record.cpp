@@ -115,8 +115,8 @@ int hipEventCreate(void** e) {
 }
 int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
 int hipEventDestroy(void*) { return 0; }
-int hipEventRecord(void*, void*) {
-  note("event");
+int hipEventRecord(void* e, void*) {
+  note("event " + std::to_string(reinterpret_cast<uintptr_t>(e)));
   return 0;
 }
 int hipEventSynchronize(void*) { return 0; }
