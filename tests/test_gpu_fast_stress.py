@@ -97,3 +97,112 @@ def test_fast_step_is_the_ordered_step(dim, scheme, shear, n):
         d = np.abs(a[f] - b[f]).reshape(n, -1).max(1) / scale
         assert d.max() <= 1e-10, (f, d.max())
         assert np.mean(d <= 1e-12) >= 0.995, (f, np.sort(d)[-4:])
+
+
+def _one_step(coords, cells, state, materials, scheme, iso=False, vu="flip", g=9.81):
+    from mpm_amd.capi import Solver
+    out = {}
+    for ordered in (True, False):
+        s = Solver(3, scheme, vu, ordered=ordered)
+        s.set_mesh(coords, cells, isoparametric=iso)
+        s.set_materials(materials)
+        s.set_gravity([0.0, 0.3 * g, -g])
+        s.set_particles(**state)
+        s.step(1, 2e-5)
+        out[ordered] = s.particles()
+        s.close()
+    return out[True], out[False]
+
+
+def _compare(a, b, extra=0.0):
+    n = len(a["x"])
+    assert np.array_equal(a["cell"], b["cell"])
+    assert np.array_equal(a["statevars"][:, 0], b["statevars"][:, 0])
+    for f in FIELDS:
+        scale = max(float(np.abs(a[f]).max()), 1e-300)
+        d = np.abs(a[f] - b[f]).reshape(n, -1).max(1) / scale
+        assert d.max() <= 1e-10 + extra, (f, d.max())
+        assert np.mean(d <= 1e-12 + extra) >= 0.995, (f, np.sort(d)[-4:])
+
+
+# Box cells of three different sides: a side or a component taken for another
+# shows. One node moved by 3 % of a side: no cell is treated as a box then (the
+# flag is the mesh's), and the general kernels run on a Cartesian mesh.
+@pytest.mark.parametrize("scheme", ["usf", "usl", "musl"])
+@pytest.mark.parametrize("vu", ["flip", "apic"])
+@pytest.mark.parametrize("move", [False, True])
+def test_unequal_sides(scheme, vu, move):
+    h = np.array([0.1, 0.07, 0.13])
+    coords, cells, state = _state(3, 1000, False, seed=5)
+    coords, state["x"] = coords / 0.1 * h, state["x"] / 0.1 * h
+    state["volume"] = state["volume"] / 0.1**3 * h.prod()
+    state["mass"] = state["volume"] * state["density"]
+    if move:
+        centre = int(np.argmin(np.abs(coords - coords.mean(0)).sum(1)))
+        coords[centre] += 0.03 * h * np.array([1.0, -1.0, 1.0])
+    a, b = _one_step(coords, cells, state, _materials(), scheme, vu=vu)
+    _compare(a, b)
+
+
+# Coordinates far from the origin. Sides of 1/16 m, an offset of 2^17 m and
+# positions on a grid of 2^-30 m are exact in 64 bits, so the step there is the
+# step at the origin but for rounding of the coordinates' products: the Jacobian
+# of 8 products of offset size, 8 * 2^-53 * 2^17 / (1 / 32) of its entries in
+# ordered mode, which the return mappings magnify by up to 10. The boxes' sides
+# do not see the offset: fast mode is no further from the step at the origin
+# than ordered mode.
+@pytest.mark.parametrize("scheme", ["usf", "usl", "musl"])
+def test_large_coordinates(scheme):
+    h, off = 0.0625, 2.0**17
+    coords, cells, state = _state(3, 600, False, seed=6)
+    coords = np.round(coords / 0.1) * h
+    state["x"] = np.round(state["x"] / 0.1 * h * 2.0**30) / 2.0**30
+    at0, _ = _one_step(coords, cells, state, _materials(), scheme)
+    state["x"] = state["x"] + off
+    a, b = _one_step(coords + off, cells, state, _materials(), scheme)
+    assert np.array_equal(a["cell"], b["cell"])
+    bound = 10 * 8 * 2.0**-53 * off * 32
+    for f in ("v", "stress", "strain", "F", "volume"):
+        scale = max(float(np.abs(at0[f]).max()), 1e-300)
+        ea, eb = (float(np.abs(q[f] - at0[f]).max()) / scale for q in (a, b))
+        assert ea <= bound and eb <= bound, (f, ea, eb, bound)
+        assert eb <= ea + 1e-10, (f, ea, eb)
+
+
+# Softening and separation. Plastic strains below, between and above the peak
+# and residual ones, in materials with and without tension cutoff, and particles
+# below the critical density.
+@pytest.mark.parametrize("scheme", ["usf", "usl", "musl"])
+@pytest.mark.parametrize("n", [129, 1000])
+def test_softened_and_separated_particles(scheme, n):
+    soft = dict(residual_friction=25.0, residual_dilation=1.0, residual_cohesion=100.0,
+                peak_pdstrain=1e-3, residual_pdstrain=1e-2, softening=True,
+                packing_fraction=0.6, packing_fraction_minimum=0.5)
+    materials = np.stack([
+        mat.mohr_coulomb(4e6, 0.3, 1900.0, friction=32.0, dilation=3.0, cohesion=500.0, **soft),
+        mat.linear_elastic(4e6, 0.25, 1700.0),
+        mat.mohr_coulomb(3e6, 0.2, 2000.0, friction=35.0, dilation=5.0, cohesion=800.0,
+                         tension_cutoff=1200.0, **soft),
+        mat.mohr_coulomb(3e6, 0.2, 2000.0, friction=35.0, dilation=5.0, cohesion=800.0,
+                         tension_cutoff=300.0, packing_fraction=0.6,
+                         packing_fraction_minimum=0.5)])
+    coords, cells, state = _state(3, n, False, seed=7)
+    r = np.random.default_rng(8)
+    mid = state["material_id"]
+    rho = materials[mid, 1] * np.where(np.arange(n) % 11 == 3, 0.8, 1.0)
+    pds = r.choice([0.0, 5e-4, 2e-3, 9e-3, 1e-2, 3e-2], n)
+    sv = np.zeros((n, mat.NSTATEVARS))
+    sv[:, 1:5] = np.stack([np.radians(materials[mid, 4]), np.radians(materials[mid, 5]),
+                           materials[mid, 6], materials[mid, 12]], 1)
+    sv[:, 8] = pds
+    state.update(density=rho, mass=state["volume"] * rho, statevars=sv)
+    a, b = _one_step(coords, cells, state, materials, scheme)
+    y, mc = a["statevars"][:, 0], materials[mid, 0] == 1
+    between = (pds > 1e-3) & (pds < 1e-2) & mc & (mid != 3)
+    assert np.any(y == 3)
+    assert np.any(between & (y == 1)) and np.any(between & (y == 2))  # a softening modulus
+    assert np.any((pds >= 1e-2) & (mid == 0) & (y == 1))              # residual strength
+    assert np.any(np.abs(a["statevars"][between, 1] - sv[between, 1]) > 1e-3)
+    cut = between & (mid == 2)
+    assert np.any(a["statevars"][cut, 4] < 1200.0)  # the apex of the softened cone
+    _compare(a, b)
