@@ -417,80 +417,70 @@ MPMX_DEV bool predictor(const Material& m, double* s, const double* ds, double d
 // Velocity gradient L (L[a][b] = d v_a / d x_b) at xi and divergence at the
 // centroid on a box cell with sides len, axis by axis: differences and sums
 // along x, interpolated over y and z. 24 node velocities, no node coordinates.
-template <int D>
-MPMX_DEV void box_gradient(const double* xi, const double* len, const double (*nv)[D],
-                           double (*L)[D], double* div_c) {
+MPMX_DEV void box_gradient(const double* xi, const double* len, const double (*nv)[3],
+                           double (*L)[3], double* div_c) {
 #pragma clang fp contract(fast)
-  double il[D];
+  double il[3];
 #pragma unroll
-  for (int k = 0; k < D; ++k) il[k] = rcp(len[k]);
+  for (int k = 0; k < 3; ++k) il[k] = rcp(len[k]);
   double dc = 0.;
 #pragma unroll
-  for (int a = 0; a < D; ++a) {
-    if constexpr (D == 2) {
-      const double d0 = nv[1][a] - nv[0][a], d1 = nv[2][a] - nv[3][a];
-      const double e0 = nv[3][a] - nv[0][a], e1 = nv[2][a] - nv[1][a];
-      L[a][0] = 0.5 * il[0] * ((d0 + d1) + xi[1] * (d1 - d0));
-      L[a][1] = 0.5 * il[1] * ((e0 + e1) + xi[0] * (e1 - e0));
-      dc = dc + (a == 0 ? 0.5 * il[0] * (d0 + d1) : 0.5 * il[1] * (e0 + e1));
-    } else {
-      // rows along x at (y, z) = 00, 10, 01, 11
-      const double d0 = nv[1][a] - nv[0][a], d1 = nv[2][a] - nv[3][a];
-      const double d2 = nv[5][a] - nv[4][a], d3 = nv[6][a] - nv[7][a];
-      const double s0 = nv[1][a] + nv[0][a], s1 = nv[2][a] + nv[3][a];
-      const double s2 = nv[5][a] + nv[4][a], s3 = nv[6][a] + nv[7][a];
-      const double m0 = s0 + xi[0] * d0, m1 = s1 + xi[0] * d1;
-      const double m2 = s2 + xi[0] * d2, m3 = s3 + xi[0] * d3;
-      const double a0 = (d0 + d1) + xi[1] * (d1 - d0), a1 = (d2 + d3) + xi[1] * (d3 - d2);
-      const double b0 = m1 - m0, b1 = m3 - m2;
-      const double c0 = (m0 + m1) + xi[1] * b0, c1 = (m2 + m3) + xi[1] * b1;
-      L[a][0] = 0.25 * il[0] * ((a0 + a1) + xi[2] * (a1 - a0));
-      L[a][1] = 0.25 * il[1] * ((b0 + b1) + xi[2] * (b1 - b0));
-      L[a][2] = 0.25 * il[2] * (c1 - c0);
-      const double w = a == 0   ? (d0 + d1) + (d2 + d3)
-                       : a == 1 ? (s1 - s0) + (s3 - s2)
-                                : (s2 + s3) - (s0 + s1);
-      dc = dc + 0.25 * il[a] * w;
-    }
+  for (int a = 0; a < 3; ++a) {
+    // rows along x at (y, z) = 00, 10, 01, 11
+    const double d0 = nv[1][a] - nv[0][a], d1 = nv[2][a] - nv[3][a];
+    const double d2 = nv[5][a] - nv[4][a], d3 = nv[6][a] - nv[7][a];
+    const double s0 = nv[1][a] + nv[0][a], s1 = nv[2][a] + nv[3][a];
+    const double s2 = nv[5][a] + nv[4][a], s3 = nv[6][a] + nv[7][a];
+    const double m0 = s0 + xi[0] * d0, m1 = s1 + xi[0] * d1;
+    const double m2 = s2 + xi[0] * d2, m3 = s3 + xi[0] * d3;
+    const double a0 = (d0 + d1) + xi[1] * (d1 - d0), a1 = (d2 + d3) + xi[1] * (d3 - d2);
+    const double b0 = m1 - m0, b1 = m3 - m2;
+    const double c0 = (m0 + m1) + xi[1] * b0, c1 = (m2 + m3) + xi[1] * b1;
+    L[a][0] = 0.25 * il[0] * ((a0 + a1) + xi[2] * (a1 - a0));
+    L[a][1] = 0.25 * il[1] * ((b0 + b1) + xi[2] * (b1 - b0));
+    L[a][2] = 0.25 * il[2] * (c1 - c0);
+    const double w = a == 0   ? (d0 + d1) + (d2 + d3)
+                     : a == 1 ? (s1 - s0) + (s3 - s2)
+                              : (s2 + s3) - (s0 + s1);
+    dc = dc + 0.25 * il[a] * w;
   }
   *div_c = dc;
 }
 
 // The same on a general cell from its Jacobian at xi and the stored centroid
 // gradients.
-template <int D>
-MPMX_DEV void cell_gradient(const Mesh& M, int c, const double* xi, const double (*nv)[D],
-                            double (*L)[D], double* div_c) {
+MPMX_DEV void cell_gradient(const Mesh& M, int c, const double* xi, const double (*nv)[3],
+                            double (*L)[3], double* div_c) {
 #pragma clang fp contract(fast)
-  constexpr int NN = Elem<D>::NN;
-  double X[NN][D], Ji[D][D];
-  load_cell_X<D>(M, c, X);
-  jacobian_inverse<D>(xi, X, Ji);
-  double G[D][D];  // sum_i v_i (x) grad_i, then L = G J^-T
+  constexpr int NN = Elem<3>::NN;
+  double X[NN][3], Ji[3][3];
+  load_cell_X<3>(M, c, X);
+  jacobian_inverse<3>(xi, X, Ji);
+  double G[3][3];  // sum_i v_i (x) grad_i, then L = G J^-T
 #pragma unroll
-  for (int a = 0; a < D; ++a)
+  for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int b = 0; b < D; ++b) G[a][b] = 0.;
-  const double* dcp = M.dndx_c + (int64_t)c * NN * D;
+    for (int b = 0; b < 3; ++b) G[a][b] = 0.;
+  const double* dcp = M.dndx_c + (int64_t)c * NN * 3;
   double dc = 0.;
 #pragma unroll
   for (int i = 0; i < NN; ++i) {
-    double g[D];
-    grad_i<D>(xi, i, g);
+    double g[3];
+    grad_i<3>(xi, i, g);
 #pragma unroll
-    for (int a = 0; a < D; ++a) {
-      dc = dc + dcp[i * D + a] * nv[i][a];
+    for (int a = 0; a < 3; ++a) {
+      dc = dc + dcp[i * 3 + a] * nv[i][a];
 #pragma unroll
-      for (int b = 0; b < D; ++b) G[a][b] = G[a][b] + nv[i][a] * g[b];
+      for (int b = 0; b < 3; ++b) G[a][b] = G[a][b] + nv[i][a] * g[b];
     }
   }
 #pragma unroll
-  for (int a = 0; a < D; ++a)
+  for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int b = 0; b < D; ++b) {
+    for (int b = 0; b < 3; ++b) {
       double t = G[a][0] * Ji[b][0];
 #pragma unroll
-      for (int k = 1; k < D; ++k) t = t + G[a][k] * Ji[b][k];
+      for (int k = 1; k < 3; ++k) t = t + G[a][k] * Ji[b][k];
       L[a][b] = t;
     }
   *div_c = dc;
@@ -499,25 +489,18 @@ MPMX_DEV void cell_gradient(const Mesh& M, int c, const double* xi, const double
 // The particle fields the kinematics and the constitutive update read, loaded
 // together before any store (a later load would wait for the stores' round
 // trip: the compiler must assume they alias).
-template <int D>
 struct StressIn {
-  static constexpr int NE = D == 2 ? 3 : 6;  // strain components that change
-  double eps[NE], F[D * 3], s[6], vol, rho;
+  double eps[6], F[9], s[6], vol, rho;
   int mat;
 };
-template <int D>
-MPMX_DEV int strain_comp(int k) {
-  return (D == 2 && k == 2) ? 3 : k;
-}
-template <int D>
-MPMX_DEV void load_stress_in(const Particles& P, int64_t p, StressIn<D>& q) {
+MPMX_DEV void load_stress_in(const Particles& P, int64_t p, StressIn& q) {
   const int64_t np = P.np;
 #pragma unroll
-  for (int k = 0; k < StressIn<D>::NE; ++k) q.eps[k] = stream_ld(&P.strain[strain_comp<D>(k) * np + p]);
+  for (int k = 0; k < 6; ++k) q.eps[k] = stream_ld(&P.strain[k * np + p]);
   q.vol = stream_ld(&P.vol[p]);
   q.rho = stream_ld(&P.rho[p]);
 #pragma unroll
-  for (int k = 0; k < D * 3; ++k) q.F[k] = stream_ld(&P.F[k * np + p]);
+  for (int k = 0; k < 9; ++k) q.F[k] = stream_ld(&P.F[k * np + p]);
 #pragma unroll
   for (int k = 0; k < 6; ++k) q.s[k] = stream_ld(&P.stress[k * np + p]);
   q.mat = stream_ld(&P.mat[p]);
@@ -526,46 +509,41 @@ MPMX_DEV void load_stress_in(const Particles& P, int64_t p, StressIn<D>& q) {
 // The kinematics of the stress update (mpm_scheme.tcc:75-103; see kinematics
 // in mpmx_kernels.hip) from the velocity gradient: strain increment ds, and
 // strain, volume, density and F of particle p written.
-template <int D>
-MPMX_DEV void strain_update(const Particles& P, int64_t p, StressIn<D>& q, const double (*L)[D],
+MPMX_DEV void strain_update(const Particles& P, int64_t p, StressIn& q, const double (*L)[3],
                             double div_c, double dt, double* ds) {
 #pragma clang fp contract(fast)
   const int64_t np = P.np;
-  double R[D][D];
+  double R[3][3];
 #pragma unroll
-  for (int a = 0; a < D; ++a)
+  for (int a = 0; a < 3; ++a)
 #pragma unroll
-    for (int b = 0; b < D; ++b) {
+    for (int b = 0; b < 3; ++b) {
       double r = L[a][b] * dt;
       if (fabs(r) < 1.E-15) r = 0.;
       R[a][b] = a == b ? 1. + r : r;
     }
 #pragma unroll
-  for (int k = 0; k < 6; ++k) ds[k] = 0.;
-#pragma unroll
-  for (int k = 0; k < D; ++k) ds[k] = L[k][k];
+  for (int k = 0; k < 3; ++k) ds[k] = L[k][k];
   ds[3] = L[0][1] + L[1][0];
-  if constexpr (D == 3) {
-    ds[4] = L[1][2] + L[2][1];
-    ds[5] = L[0][2] + L[2][0];
-  }
+  ds[4] = L[1][2] + L[2][1];
+  ds[5] = L[0][2] + L[2][0];
 #pragma unroll
   for (int k = 0; k < 6; ++k) ds[k] = fabs(ds[k]) < 1.E-15 ? 0. : ds[k] * dt;
   const double dvol = dt * div_c;
   q.vol = q.vol * (1. + dvol);
   q.rho = q.rho * rcp(1. + dvol);
 #pragma unroll
-  for (int k = 0; k < StressIn<D>::NE; ++k)
-    stream_st(&P.strain[strain_comp<D>(k) * np + p], q.eps[k] + ds[strain_comp<D>(k)]);
+  for (int k = 0; k < 6; ++k)
+    stream_st(&P.strain[k * np + p], q.eps[k] + ds[k]);
   stream_st(&P.vol[p], q.vol);
   stream_st(&P.rho[p], q.rho);
 #pragma unroll
-  for (int a = 0; a < D; ++a)
+  for (int a = 0; a < 3; ++a)
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       double t = R[a][0] * q.F[j];
 #pragma unroll
-      for (int b = 1; b < D; ++b) t = t + R[a][b] * q.F[b * 3 + j];
+      for (int b = 1; b < 3; ++b) t = t + R[a][b] * q.F[b * 3 + j];
       stream_st(&P.F[(a * 3 + j) * np + p], t);
     }
 }

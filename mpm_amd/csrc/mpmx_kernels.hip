@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(CH) void k_p2g(Mesh M, Particles P, Nodes Nd, StepA
 // memory holds it.
 template <int D, bool KEEP, int BS>
 MPMX_DEV void block_stress_update(fast::Returns<BS>& R, bool live, const Particles& P,
-                                  const Material* mats, int p, fast::StressIn<D>& q,
+                                  const Material* mats, int p, fast::StressIn& q,
                                   const double (*L)[D], double div_c, double dt) {
   const int64_t np = P.np;
   const int tid = threadIdx.x;
@@ -1024,7 +1024,7 @@ MPMX_DEV void block_stress_update(fast::Returns<BS>& R, bool live, const Particl
     double sv[NSV];
     if (m.type != LE) load_sv(P, m, p, sv);
     double ds[6];
-    fast::strain_update<D>(P, p, q, L, div_c, dt, ds);
+    fast::strain_update(P, p, q, L, div_c, dt, ds);
     bool done = true;
     if (m.type == LE) {
       double t[6];
@@ -1093,9 +1093,9 @@ MPMX_DEV void velocity_gradient(const Mesh& M, int c, const double* xi, const do
     double len[D];
 #pragma unroll
     for (int k = 0; k < D; ++k) len[k] = M.len[k * M.ncells + c];
-    fast::box_gradient<D>(xi, len, nv, L, div_c);
+    fast::box_gradient(xi, len, nv, L, div_c);
   } else {
-    fast::cell_gradient<D>(M, c, xi, nv, L, div_c);
+    fast::cell_gradient(M, c, xi, nv, L, div_c);
   }
 }
 
@@ -1111,13 +1111,13 @@ __global__ __launch_bounds__(kStressBlock) MPMX_WAVES(BOX ? 3 : 2) void k_stress
   const int c = p < np ? P.cell[p] : -1;
   const bool live = valid_cell<D>(M, c);
   double L[D][D], div_c = 0., x[D];
-  fast::StressIn<D> q;
+  fast::StressIn q;
   if (live) {
     double xi[D], nv[NN][D];
 #pragma unroll
     for (int k = 0; k < D; ++k) xi[k] = P.xi[k * np + p];
     gather_nodes<D>(M, Nd, c, nv, nullptr);
-    fast::load_stress_in<D>(P, p, q);
+    fast::load_stress_in(P, p, q);
     if constexpr (LOCATE) {
 #pragma unroll
       for (int k = 0; k < D; ++k) x[k] = stream_ld(&P.x[k * np + p]);
@@ -1148,14 +1148,14 @@ __global__ __launch_bounds__(CH) MPMX_WAVES(2) void k_stress_scatter_fast(
   const int key = tid < cnt ? P.cell[p] : -1;
   const bool live = valid_cell<D>(M, key);
   double xi[D], L[D][D], div_c = 0., mass = 0.;
-  fast::StressIn<D> q;
+  fast::StressIn q;
   if (live) {
     double nv[NN][D];
 #pragma unroll
     for (int k = 0; k < D; ++k) xi[k] = P.xi[k * np + p];
     mass = P.mass[p];
     gather_nodes<D>(M, Nd, key, nv, nullptr);
-    fast::load_stress_in<D>(P, p, q);
+    fast::load_stress_in(P, p, q);
     velocity_gradient<D, BOX>(M, key, xi, nv, L, &div_c);
   }
   block_stress_update<D, true, CH>(sh.R, live, P, mats, p, q, L, div_c, A.dt);
@@ -1189,7 +1189,7 @@ __global__ __launch_bounds__(kBlock) MPMX_WAVES(2) void k_g2p_stress_fast(
   const int c = p < np ? P.cell[p] : -1;
   const bool live = valid_cell<D>(M, c);
   double L[D][D], div_c = 0.;
-  fast::StressIn<D> q;
+  fast::StressIn q;
   if (live) {
     double xi[D], N[NN], nv[NN][D], sv[D], sa[D];
 #pragma unroll
@@ -1217,7 +1217,7 @@ __global__ __launch_bounds__(kBlock) MPMX_WAVES(2) void k_g2p_stress_fast(
       x[k] = stream_ld(&P.x[k * np + p]);
       u0[k] = stream_ld(&P.u[k * np + p]);
     }
-    fast::load_stress_in<D>(P, p, q);
+    fast::load_stress_in(P, p, q);
     const int pvc = P.pvc_mask ? P.pvc_mask[p] : 0;
     const double beta = vu == ASFLIP ? P.beta[p] : 0.;
     velocity_gradient<D, BOX>(M, c, xi, nv, L, &div_c);
@@ -2268,8 +2268,8 @@ void launch_affine_matrix(const Mesh& M, const Particles& P, int vu, const Statu
 template <int D>
 void launch_locate_step(bool fast, const Mesh& M, const Particles& P, Status* S, int* scan_list,
                         hipStream_t st) {
-  if (fast)
-    MPMX_LAUNCH((k_locate_step<D, true>), P.np, st, M, P, S, scan_list);
+  if (D == 3 && fast)
+    MPMX_LAUNCH((k_locate_step<D, D == 3>), P.np, st, M, P, S, scan_list);
   else
     MPMX_LAUNCH((k_locate_step<D, false>), P.np, st, M, P, S, scan_list);
 }
