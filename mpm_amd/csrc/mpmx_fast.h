@@ -9,10 +9,10 @@
 // instead of two 6-vectors and a 6x6 product each. FP64 throughout. What the
 // Lode angle is sensitive to (j2, j3 and the two ratios formed from them, whose
 // rounding the angle magnifies by 1 / sin 3 theta) keeps the reference's
-// expressions bit for bit; against the reference's arithmetic on the same
-// inputs the returned stresses differ by 1e-14 of their size in the mean and
-// 2e-10 Pa at most over 5e5 random returns, 4 to 5 orders below what moving the
-// inputs by an ulp does.
+// expressions bit for bit; against the reference's arithmetic on 5e5 random
+// states (stresses up to 2e4 Pa) the new stresses differ by 1e-12 Pa in the mean
+// and 3e-8 Pa at most, where moving the start stress by an ulp moves the
+// reference's own result by up to 6e-6 Pa (tests/test_fast_return_host.py).
 // Collapse (2.1M particles, half of them yielding): stress update 364 + 180 us
 // (deferred return mappings, 1450 instructions a correction) -> 345 us in one
 // kernel; slope (5.2M, elastic) 702 + 19 -> 541 us, 4.3 TB/s of compulsory

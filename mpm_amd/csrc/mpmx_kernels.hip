@@ -461,8 +461,9 @@ __global__ __launch_bounds__(kBlock) void k_locate_init(Mesh M, Particles P, Sta
 
 // Per-step locate of an isoparametric mesh (the step kernels locate Cartesian
 // meshes themselves): current cell, then neighbours, else the scan queue.
-// FAST: fast mode's iteration for hex8 cells (two waves per SIMD: 0.22 ms on
-// the 254k-particle draped block against 0.34 ms at one without spills).
+// FAST: fast mode's iteration for hex8 cells (two waves per SIMD with 125
+// spilled registers: 0.22 ms on the 254k-particle draped block, against 0.34 ms
+// at one without spills).
 template <int D, bool FAST>
 __global__ __launch_bounds__(kBlock) MPMX_PRED_ATTR void k_locate_step(Mesh M, Particles P, Status* S,
                                                         int* scan_list) {
@@ -1002,8 +1003,11 @@ __global__ __launch_bounds__(CH) void k_p2g(Mesh M, Particles P, Nodes Nd, StepA
 // ----------------------- 3D fast mode: stress update -------------------------
 // Occupancy: 3 waves per SIMD for k_stress_fast on box cells (14 spilled
 // registers in the return mapping; collapse 345 us, slope 541 us, against 359
-// and 585 us at 2 waves without spills), 2 for the USF scatter (146 against
-// 160 us, 570k particles) and the general cells (92 against 132 us, 254k).
+// and 585 us at 2 waves without spills). 2 elsewhere: k_stress_fast on general
+// cells (no spills; 2.1M particles 417 us, against 685 us at 3 waves with 85),
+// the USF scatter (146 against 160 us, 570k particles) and the USL kernel (box
+// cells, no spills, 2.1M particles: 458 us, against 670 us at 3 waves with 74;
+// general cells, 254k: 91 us with 84 spills, against 131 us with 168).
 // The stress update of a workgroup of BS particles (every thread calls it;
 // `live`: the thread has a particle p in a cell, its fields loaded and its
 // velocity gradient formed): kinematics, elastic predictor, and the return
@@ -1921,7 +1925,7 @@ MPMX_DEV void gather_terms(const Mesh& M, const Particles& P, int64_t n, int p, 
 }
 
 // Waves per SIMD of the gathers: the 3D sums of all quantities gain from 5 (128
-// us against 132) and MUSL's second momentum, which takes its ranks ready-made,
+// us, with 12 spilled registers, against 132) and MUSL's second momentum, which takes its ranks ready-made,
 // from 7, as do the 2D ones (16.0 us against 17.8 at 6400 particles); USF's
 // two 3D ones are best as the compiler has them (262k particles:
 // 74 / 105 us, at 5 waves 83 / 120).
