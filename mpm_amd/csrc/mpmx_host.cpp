@@ -229,7 +229,8 @@ struct mpmx_ctx {
   // staging of the particle read-back (read_rows)
   DBuf<char> d_read;
   char* h_read = nullptr;  // pinned
-  size_t read_bytes = 0;   // of each of the two halves
+  size_t read_bytes = 0;   // of each of the two pinned halves (d_read holds two as well)
+  double read_lost = 0.;   // us lost by large reads without them
   bool was_read = false;
   hipEvent_t read_done[2] = {nullptr, nullptr};
 
@@ -756,111 +757,116 @@ struct ReadField {
   int comps, kind, size;
 };
 
-// The array's components one by one, transposed on the host.
-template <class T, class R>
-void read_components(const ReadField& f, int64_t n, hipStream_t st) {
-  std::vector<T> col(n);
-  R* rows = (R*)f.out;
-  for (int k = 0; k < f.comps; ++k) {
-    HIPCHECK(hipMemcpyAsync(col.data(), (const T*)f.in + (size_t)k * n, n * sizeof(T),
-                            hipMemcpyDeviceToHost, st));
-    HIPCHECK(hipStreamSynchronize(st));
-    for (int64_t i = 0; i < n; ++i) rows[i * f.comps + k] = col[i];
+// A run of rows of one field, packed at `off` of the staging.
+struct ReadPiece {
+  const ReadField* f;
+  int64_t r0, rows;
+  size_t off;
+};
+
+// Packs rows of the fields from row r0 of field k on into `room` bytes at
+// `dev`, as many as fit; moves (k, r0) past them and returns the bytes used.
+size_t pack_rows(mpmx_ctx* c, const std::vector<ReadField>& f, int64_t n, size_t& k, int64_t& r0,
+                 char* dev, size_t room, std::vector<ReadPiece>& pieces) {
+  PackTable T;
+  T.count = 0;
+  size_t used = 0;
+  pieces.clear();
+  while (k < f.size() && T.count < PackTable::kMax && used < room) {
+    const size_t row = (size_t)f[k].comps * f[k].size;
+    const int64_t rows = std::min<int64_t>(n - r0, (int64_t)((room - used) / row));
+    if (rows <= 0) break;
+    T.e[T.count++] = {f[k].in, dev + used, r0, rows, f[k].comps, f[k].kind};
+    pieces.push_back({&f[k], r0, rows, used});
+    used = (used + rows * row + 15) & ~size_t(15);
+    r0 += rows;
+    if (r0 < n) break;
+    r0 = 0;
+    ++k;
   }
+  launch_pack_rows(T, n, c->stream);
+  HIPCHECK(hipGetLastError());
+  return used;
 }
 
-// Copies fields of n particles to the host: packed into rows by a kernel, a
-// piece of the staging at a time, each piece one copy to pinned memory while
-// the piece before it is spread to the caller's arrays. (A copy per component
-// and a transposition on the host took 0.5 ms for 8192 particles, most of it
-// the 63 copies' latency.) The staging, twice the size of the largest read so
-// far and at most 2 x 4 MiB on each side, stays the context's.
-// A context's first read makes the staging, up to 2 ms of fresh pinned pages.
-// Where that is more than the first read gains, which may be the only one, the
-// components are copied one by one: few of them, and neither so little data
-// that the staging costs nothing nor so much that one read pays for it. x and
-// v, first read with copies / with the staging made / later reads: 512
-// particles 93 / 67 / 24 us, 8192 67 / 86 / 49, 24k 110 / 145 / 75, 111k 410 /
-// 455 to 2400 / 270, 262k (3D) 1800 / 980 to 4400 / 740, 2M (3D) 16400 / 9900 /
-// 6200; all 63 components of 8192 particles 660 / 270 / 200.
-constexpr int kFirstReadCopies = 8;
-constexpr size_t kFirstReadMin = size_t(128) << 10, kFirstReadMax = size_t(32) << 20;
+// Copies fields of n particles to the host, packed into rows by a kernel, a
+// piece of at most 4 MiB of the staging at a time. (A copy per component and a
+// transposition on the host took 0.5 ms for 8192 particles, most of it the 63
+// copies' latency.) Two ways from there:
+//  * one copy per piece to pinned memory, spread to the caller's arrays while
+//    the next piece is on its way. Its fresh pinned pages, 2 x up to 4 MiB, cost
+//    1 to 3 ms once a context where a read takes more than 1 MiB.
+//  * for one or two fields, one copy each straight to the caller's arrays: as
+//    fast up to a piece, 22 us a MiB slower beyond (and slower than pinned, as
+//    copies per component, for a process's first some 10 to 50). Taken for a
+//    context's first read, for all reads of 1 to 4 MiB, and for larger ones until
+//    what they lose reaches the staging's cost.
+// us a read of a context's first / second / later, copies per component - pinned
+// - as here: x and v of 8192 particles 69 58 58 - 86 51 49 - 54 75 49, 111k 422
+// 364 324 - 455 (2380 in a process's second context) 291 270 - 392 302 283, 262k
+// (3D) 1766 1680 1533 - 980 (4400) 820 750 - 1235 1075 750 from the 6th on.
+constexpr size_t kReadPiece = size_t(4) << 20;
+constexpr size_t kReadSmall = size_t(128) << 10;
 void read_rows(mpmx_ctx* c, const std::vector<ReadField>& f, int64_t n) {
   if (f.empty()) return;
-  size_t want = size_t(64) << 10, total = 0;
-  int copies = 0;
-  for (const auto& q : f) {
-    total += (size_t)q.comps * q.size * n + 16;
-    copies += q.comps;
-  }
+  const size_t grain = size_t(64) << 10;
+  size_t want = grain, total = 0;
+  for (const auto& q : f) total += (size_t)q.comps * q.size * n + 16;
+  while (want < total && want < kReadPiece) want *= 2;
   const bool first = !c->was_read;
   c->was_read = true;
-  if (first && copies <= kFirstReadCopies && total >= kFirstReadMin && total <= kFirstReadMax) {
-    for (const auto& q : f) {
-      if (q.kind == PACK_F64)
-        read_components<double, double>(q, n, c->stream);
-      else if (q.kind == PACK_I32)
-        read_components<int, int>(q, n, c->stream);
-      else
-        read_components<int, int64_t>(q, n, c->stream);
+  bool direct = f.size() <= 2 && total >= kReadSmall;
+  if (direct && want <= (size_t(1) << 20)) {
+    direct = first;
+  } else if (direct && total > kReadPiece) {
+    const double mib = 1. / (1 << 20), loss = 22. * (total - kReadPiece) * mib;
+    direct = c->read_bytes < want && c->read_lost + loss <= 250. * (want * mib);
+    if (direct) c->read_lost += loss;
+  }
+  size_t k = 0;
+  int64_t r0 = 0;
+  if (direct) {
+    const size_t room = std::min((total + grain - 1) / grain * grain, kReadPiece);
+    if (c->d_read.n < room) c->d_read.alloc(room);
+    std::vector<ReadPiece> pieces;
+    while (k < f.size()) {
+      pack_rows(c, f, n, k, r0, c->d_read.p, room, pieces);
+      for (const ReadPiece& p : pieces) {
+        const size_t row = (size_t)p.f->comps * p.f->size;
+        HIPCHECK(hipMemcpyAsync(p.f->out + p.r0 * row, c->d_read.p + p.off, p.rows * row,
+                                hipMemcpyDeviceToHost, c->stream));
+      }
+      HIPCHECK(hipStreamSynchronize(c->stream));
     }
     return;
   }
-  while (want < total && want < (size_t(4) << 20)) want *= 2;
   if (c->read_bytes < want) {
     if (c->h_read) (void)hipHostFree(c->h_read);
     c->h_read = nullptr;
     c->read_bytes = 0;
-    c->d_read.alloc(2 * want);
+    if (c->d_read.n < 2 * want) c->d_read.alloc(2 * want);
     HIPCHECK(hipHostMalloc((void**)&c->h_read, 2 * want));
     c->read_bytes = want;
     for (auto& e : c->read_done)
       if (!e) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
   const size_t side_bytes = c->read_bytes;
-  struct Piece {
-    const ReadField* f;
-    int64_t r0, rows;
-    size_t off;
-  };
-  std::vector<Piece> pieces[2];
+  std::vector<ReadPiece> pieces[2];
   auto spread = [&](int side) {
     if (pieces[side].empty()) return;
     HIPCHECK(hipEventSynchronize(c->read_done[side]));
-    for (const Piece& p : pieces[side]) {
+    for (const ReadPiece& p : pieces[side]) {
       const size_t row = (size_t)p.f->comps * p.f->size;
       std::memcpy(p.f->out + p.r0 * row, c->h_read + side * side_bytes + p.off, p.rows * row);
     }
     pieces[side].clear();
   };
-  size_t k = 0;
-  int64_t r0 = 0;
   for (int side = 0; k < f.size(); side ^= 1) {
     spread(side);
-    PackTable T;
-    T.count = 0;
-    size_t used = 0;
-    while (k < f.size() && T.count < PackTable::kMax) {
-      const size_t row = (size_t)f[k].comps * f[k].size;
-      const int64_t rows = std::min<int64_t>(n - r0, (int64_t)((side_bytes - used) / row));
-      if (rows <= 0) break;
-      T.e[T.count++] = {f[k].in, c->d_read.p + side * side_bytes + used, r0, rows, f[k].comps,
-                        f[k].kind};
-      pieces[side].push_back({&f[k], r0, rows, used});
-      used = (used + rows * row + 15) & ~size_t(15);
-      r0 += rows;
-      if (r0 < n || used >= side_bytes) break;
-      r0 = 0;
-      ++k;
-    }
-    if (r0 == n) {
-      r0 = 0;
-      ++k;
-    }
-    launch_pack_rows(T, n, c->stream);
-    HIPCHECK(hipGetLastError());
-    HIPCHECK(hipMemcpyAsync(c->h_read + side * side_bytes, c->d_read.p + side * side_bytes, used,
-                            hipMemcpyDeviceToHost, c->stream));
+    char* dev = c->d_read.p + side * side_bytes;
+    const size_t used = pack_rows(c, f, n, k, r0, dev, side_bytes, pieces[side]);
+    HIPCHECK(hipMemcpyAsync(c->h_read + side * side_bytes, dev, used, hipMemcpyDeviceToHost,
+                            c->stream));
     HIPCHECK(hipEventRecord(c->read_done[side], c->stream));
   }
   spread(0);

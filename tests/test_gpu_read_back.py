@@ -45,10 +45,11 @@ def test_fields_come_back_as_set(dim, n, mc):
         assert np.array_equal(some[f], got[f]), f
 
 
-# A context's first read of few components is copied as it lies, later and
-# other ones are packed; a read beyond the staging held so far makes a larger
-# one (8192 particles in one piece of 3 MB, 30000 in three of 4 MiB).
-@pytest.mark.parametrize("dim,n", [(2, 1), (3, 257), (2, 8192), (3, 30000)])
+# One or two fields go straight to the arrays on a first read and where they take
+# 1 to 4 MiB (or more, before the staging is made), others through pinned
+# staging, which grows with them: 8192 particles in one piece of 3 MB, 30000 in
+# three of 4 MiB, x and v of 120001 in 3D in two.
+@pytest.mark.parametrize("dim,n", [(2, 1), (3, 257), (2, 8192), (3, 30000), (3, 120001)])
 def test_reads_of_one_context_agree(dim, n):
     from mpm_amd.capi import Solver
     r = np.random.default_rng(n)
