@@ -1530,9 +1530,18 @@ void remove_lost_particles(mpmx_ctx* c) {
   c->invalidate_graph();
 }
 
+// Fail if a particle left the mesh in the run whose status was read
+// (locate_particles, mpm_scheme.tcc:250-256).
+void require_located(const mpmx_ctx* c) {
+  if (c->h_status->first_bad_step != std::numeric_limits<int64_t>::max())
+    throw ApiError(MPMX_E_UNLOCATABLE,
+                   "Particle(s) outside the mesh domain: " + std::to_string(c->h_status->bad_particle) +
+                       " (step " + std::to_string(c->h_status->first_bad_step) + ")");
+}
+
 // Wait for the queued steps; take the step counter; fail if a particle left
-// the mesh (locate_particles, mpm_scheme.tcc:250-256), or, in remove mode,
-// remove the particles that did (mpm_scheme.tcc:258-260).
+// the mesh, or, in remove mode, remove the particles that did
+// (mpm_scheme.tcc:258-260).
 void check_status(mpmx_ctx* c) {
   read_status(c);
   c->step = c->h_status->step;
@@ -1540,10 +1549,7 @@ void check_status(mpmx_ctx* c) {
                     c->h_status->first_bad_step == std::numeric_limits<int64_t>::max();
   c->status_step = c->step;
   if (c->h_status->nlost > 0) remove_lost_particles(c);
-  if (c->h_status->first_bad_step != std::numeric_limits<int64_t>::max())
-    throw ApiError(MPMX_E_UNLOCATABLE,
-                   "Particle(s) outside the mesh domain: " + std::to_string(c->h_status->bad_particle) +
-                       " (step " + std::to_string(c->h_status->first_bad_step) + ")");
+  require_located(c);
 }
 
 // ------------------------ step without allocation ----------------------------
@@ -2653,7 +2659,10 @@ int mpmx_autotune(mpmx_ctx* c, double dt, double damping_factor, int trial_steps
             launch_steps(c, steps, dt, damping_factor);
           }
           HIPCHECK(hipEventRecord(e1, c->stream));
-          check_status(c);
+          // particles that left the mesh in remove mode come back with the
+          // state: they have lost their cell only
+          read_status(c);
+          require_located(c);
           float ms = 0.f;
           HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
           if (first || ms < best_ms) {

@@ -83,3 +83,21 @@ def test_autotune_ordered_mode_is_a_no_op():
     s = w.setup(Solver(2, "usf", ordered=True))
     assert s.autotune(w.dt, trial_steps=2) == dict(chunk=256, sort_every=8)
     s.close()
+
+
+def test_autotune_keeps_particles_that_its_trials_lose():
+    """In remove mode a particle that leaves the mesh within the trial steps is
+    back with the restored state, and leaves in the run."""
+    import lost_particle_deck as deck
+    from mpm_amd.capi import Solver
+    s = deck.setup(Solver(2, "usl"))
+    s.set_locate_particles(False)
+    s.step(10, deck.DT)
+    before, n = s.particles(), s.nparticles
+    s.autotune(deck.DT, trial_steps=60)
+    after = s.particles()
+    assert s.nparticles == n and s.step_count == 10
+    for f in FIELDS + ("cell", "statevars"):
+        assert np.array_equal(before[f], after[f]), f
+    s.step(60, deck.DT)
+    assert s.nparticles == n - 1
