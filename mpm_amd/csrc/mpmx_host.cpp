@@ -750,6 +750,22 @@ void get_soa(const DBuf<T>& b, int64_t np, int comps, T* rows, hipStream_t st) {
   }
 }
 
+// The context's device made current for a while: reading state back copies on
+// the context's stream, which any current device allowed, and also allocates and
+// launches.
+struct CurrentDevice {
+  int before = 0, now;
+  explicit CurrentDevice(int device) : now(device) {
+    HIPCHECK(hipGetDevice(&before));
+    if (before != now) HIPCHECK(hipSetDevice(now));
+  }
+  ~CurrentDevice() {
+    if (before != now) (void)hipSetDevice(before);
+  }
+  CurrentDevice(const CurrentDevice&) = delete;
+  CurrentDevice& operator=(const CurrentDevice&) = delete;
+};
+
 // One array to read back: component-major on the device, rows on the host.
 struct ReadField {
   const void* in;
@@ -2458,6 +2474,7 @@ int mpmx_get_particles(mpmx_ctx* c, double* x, double* u, double* v, double* str
     add(c->d_sv.p, statevars, NSV);
   else if (statevars)
     std::fill(statevars, statevars + np * NSV, 0.0);
+  const CurrentDevice device(c->device);
   read_rows(c, f, np);
   API_END(c)
 }

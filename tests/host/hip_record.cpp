@@ -14,6 +14,7 @@ std::string& g_log = *new std::string;
 std::map<const void*, std::string>& g_names = *new std::map<const void*, std::string>;
 std::map<void*, size_t>& g_size = *new std::map<void*, size_t>;
 size_t g_device = 0, g_pinned = 0;  // bytes held now
+int g_current = 0;                  // of two devices
 bool g_capturing = false;
 int g_handles = 0;
 
@@ -57,7 +58,8 @@ int __hipPopCallConfiguration(Dim3* g, Dim3* b, size_t* shared, void** stream) {
   return 0;
 }
 int hipLaunchKernel(const void* f, Dim3, Dim3, void**, size_t, void*) {
-  note((g_capturing ? "captured " : "launch ") + g_names[f]);
+  note((g_capturing ? "captured " : "launch ") + g_names[f] +
+       (g_current ? " on the other device" : ""));
   return 0;
 }
 
@@ -65,7 +67,7 @@ int hipMalloc(void** p, size_t n) {
   *p = std::calloc(n ? n : 1, 1);
   g_size[*p] = n;
   g_device += n;
-  note("malloc " + std::to_string(n));
+  note("malloc " + std::to_string(n) + (g_current ? " on the other device" : ""));
   return *p ? 0 : 2;
 }
 int hipFree(void* p) {
@@ -125,11 +127,15 @@ int hipEventElapsedTime(float* ms, void*, void*) {
   return 0;
 }
 int hipGetDevice(int* d) {
-  *d = 0;
+  *d = g_current;
+  return 0;
+}
+int hipSetDevice(int d) {
+  g_current = d;
   return 0;
 }
 int hipGetDeviceCount(int* n) {
-  *n = 1;
+  *n = 2;
   return 0;
 }
 const char* hipGetErrorString(int) { return "recorded"; }

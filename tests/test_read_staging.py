@@ -90,3 +90,23 @@ assert len([l for l in calls if l.startswith("pinned")]) == 1, calls
 print("ok")
 """ % (dim, n, fields))
     assert "ok" in out
+
+
+@pytest.mark.parametrize("n,fields", [(512, ["x", "v"]), (24000, ["x", "v"]), (8192, None)])
+def test_reads_with_another_device_current(lib, n, fields):
+    """The staging and its kernel are the context's device's, whichever is
+    current, and the caller's current device stays."""
+    out = hip_record.run(lib, """
+s = solver(3, "usl", %d)
+fields = %r
+rec.hipSetDevice(1)
+s.particles(fields) if fields else s.particles()
+calls = log()
+assert any("k_pack_rows" in l for l in calls)
+assert not [l for l in calls if "other device" in l], calls
+d = ctypes.c_int(-1)
+rec.hipGetDevice(ctypes.byref(d))
+assert d.value == 1
+print("ok")
+""" % (n, fields))
+    assert "ok" in out
